@@ -843,37 +843,40 @@ __device__ __forceinline__ void cell_terms(const DevMesh &m, const DevState &s, 
   using F = Flow<FLOW>;
   const Consts k = case_consts<B>(m, k_, c);
   const int nc = m.nc;
+  // the cell's faces in ascending order, each added with the cell's sign
+  // (left +, right -): the reference's scatter order.  Sums are FP64 in every
+  // mode.  A cell has three or four faces; an empty fourth slot reads the
+  // third face again and adds -0.0, which leaves every sum's bits as they
+  // are.  So no load waits for a branch: the face ids come in one round trip
+  // and the whole record of the four faces in the next, where a loop with a
+  // branch per face waited for each face in turn (and held the ids in LDS
+  // for Euler).  Bound by these two latencies on small meshes, by its
+  // traffic on large ones.  Measured: Euler 20 k cells 10.4 -> 3.6 us, 106 k
+  // 20.7 -> 5.9 us; laminar 100 k (batch) 10.0 -> 8.0 us; SST 1 M 99.9 ->
+  // 97.3 us, 245 k mixed 16.7 -> 14.4 us.
   int fs[4];
-  int ns = 0;
-  for (int sl = 0; sl < 4; sl++) {
-    int e = m.cf[sl * nc + c];
-    if (e == kNoSlot) break;
-    fs[ns++] = e;
-  }
-  // faces in ascending order, each added with this cell's sign (left +,
-  // right -): the reference's scatter order.  Sums are FP64 in every mode.
+#pragma unroll
+  for (int i = 0; i < 4; i++) fs[i] = m.cf[i * nc + c];
+  const bool four = fs[3] != kNoSlot;
+  if (!four) fs[3] = fs[2];
+  auto term = [&](int i, double v, bool minus) {
+    const double x = (fs[i] < 0) != minus ? -v : v;
+    return i < 3 || four ? x : -0.0;
+  };
   using RP = RecPairs<FLOW>;
   double Rc[4] = {0, 0, 0, 0};
-  for (int i = 0; i < ns; i++) {
-    const int e = fs[i];
-    const double2 a = in.pair(i, e, RP::conv0), b = in.pair(i, e, RP::conv1);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const double2 a = in.pair(i, fs[i], RP::conv0), b = in.pair(i, fs[i], RP::conv1);
     const double v[4] = {a.x, a.y, b.x, b.y};
-    if (e >= 0) {
-      for (int j = 0; j < 4; j++) Rc[j] += v[j];
-    } else {
-      for (int j = 0; j < 4; j++) Rc[j] -= v[j];
-    }
+    for (int j = 0; j < 4; j++) Rc[j] += term(i, v[j], false);
   }
   if (F::visc) {
-    for (int i = 0; i < ns; i++) {
-      const int e = fs[i];
-      const double2 a = in.pair(i, e, RP::visc0), b = in.pair(i, e, RP::visc1);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const double2 a = in.pair(i, fs[i], RP::visc0), b = in.pair(i, fs[i], RP::visc1);
       const double v[4] = {a.x, a.y, b.x, b.y};
-      if (e >= 0) {
-        for (int j = 0; j < 4; j++) Rc[j] -= v[j];
-      } else {
-        for (int j = 0; j < 4; j++) Rc[j] += v[j];
-      }
+      for (int j = 0; j < 4; j++) Rc[j] += term(i, v[j], true);
     }
   }
   const double V = m.vol[c];
@@ -884,10 +887,12 @@ __device__ __forceinline__ void cell_terms(const DevMesh &m, const DevState &s, 
       Rc[j] += V * (k.dts[0] * s.W[pidx(j, nc, c)] + k.dts[1] * s.Wt1[pidx(j, nc, c)] + k.dts[2] * s.Wt2[pidx(j, nc, c)]);
   }
   double lamc = 0, lamv = 0;
-  for (int i = 0; i < ns; i++) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
     const double2 l = in.pair(i, fs[i], RP::lam);
-    lamc += l.x;
-    if (F::visc) lamv += l.y / V;
+    const bool has = i < 3 || four;
+    lamc += has ? l.x : -0.0;
+    if (F::visc) lamv += has ? l.y / V : -0.0;
   }
   const double OMEGAN = 1.5;
   double dtc;
@@ -922,16 +927,11 @@ __device__ __forceinline__ void cell_terms(const DevMesh &m, const DevState &s, 
     double Q1 = Cw * rho * P / mutc - beta * rho * w * w + 2 * (1 - F1c) * rho * SST_SW2 / w * rdiv;
     trc[0] = -(Q0 * V);
     trc[1] = -(Q1 * V);
-    for (int i = 0; i < ns; i++) {
-      const int e = fs[i];
-      const double2 t = in.pair(i, e, RP::sst);
-      if (e >= 0) {
-        trc[0] += t.x;
-        trc[1] += t.y;
-      } else {
-        trc[0] -= t.x;
-        trc[1] -= t.y;
-      }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const double2 t = in.pair(i, fs[i], RP::sst);
+      trc[0] += term(i, t.x, false);
+      trc[1] += term(i, t.y, false);
     }
     // SSTkomegaModel::SolveDiag
     double diagt = V / dtc + 0.5 * OMEGAN * lamc + lamv;
