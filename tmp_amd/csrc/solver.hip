@@ -1094,66 +1094,99 @@ struct NormBlocks {
   int *ctr = nullptr;
 };
 
-// DF of one dependency neighbour nb of cell c across slot sl (SolveDF,
-// TopologyHolderStrategy.cpp:217-323; SST SolveDF, SSTKWStrategy.h:251-417),
-// given nb's increments (dW1 in the forward sweep, dW in the backward one):
-// the term t that the cell's sum adds.
+// What DF of one dependency neighbour reads besides the neighbour's
+// increments: its state, the face's normal and length, and r_A.
 template <int FLOW>
-__device__ __forceinline__ void df_term(const DevMesh &m, const DevState &s, int c, int sl, bool left, int nb,
-                                        const double *dW, const double *tdw, double *t, double *tt) {
-  using F = Flow<FLOW>;
-  const int nc = m.nc;
-  const size_t sc = (size_t)sl * nc + c;
-  const double n0 = m.snx[sc], n1 = m.sny[sc], A = m.sA[sc];
-  double W[4], Wp[4], Fc[4], Fcp[4];
-  for (int j = 0; j < 4; j++) {
-    const double W0 = s.W[pidx(j, nc, nb)];
-    Wp[j] = W0 + dW[j];
-    W[j] = W0;
+struct DfLoads {
+  double W[4], n0, n1, A, rA, tw[2];
+  __device__ __forceinline__ void load(const DevMesh &m, const DevState &s, int c, int sl, int nb) {
+    const size_t sc = (size_t)sl * m.nc + c;
+    load4p(s.W, m.nc, nb, W);
+    n0 = m.snx[sc];
+    n1 = m.sny[sc];
+    A = m.sA[sc];
+    rA = s.rA[sc];
+    if (Flow<FLOW>::sst) {
+      const double2 t = ld2(s.tW, 0, m.nc, nb);
+      tw[0] = t.x;
+      tw[1] = t.y;
+    }
   }
-  cons_flux(W, n0, n1, Fc);
-  cons_flux(Wp, n0, n1, Fcp);
-  const double rA = s.rA[sc];
+};
+
+// DF of one dependency neighbour (SolveDF, TopologyHolderStrategy.cpp:217-323;
+// SST SolveDF, SSTKWStrategy.h:251-417), given the neighbour's increments
+// (dW1 in the forward sweep, dW in the backward one): the term t that the
+// cell's sum adds.
+template <int FLOW>
+__device__ __forceinline__ void df_term(const DfLoads<FLOW> &l, bool left, const double *dW, const double *tdw,
+                                        double *t, double *tt) {
+  using F = Flow<FLOW>;
+  double Wp[4], Fc[4], Fcp[4];
+  for (int j = 0; j < 4; j++) Wp[j] = l.W[j] + dW[j];
+  cons_flux(l.W, l.n0, l.n1, Fc);
+  cons_flux(Wp, l.n0, l.n1, Fcp);
   for (int j = 0; j < 4; j++) {
     double DFc = left ? (Fcp[j] - Fc[j]) : (Fc[j] - Fcp[j]);
-    double Fv = rA * dW[j];
-    t[j] = 0.5 * (DFc - Fv) * A;
+    double Fv = l.rA * dW[j];
+    t[j] = 0.5 * (DFc - Fv) * l.A;
   }
   if (F::sst) {
-    double u = W[2] / W[0], v = W[3] / W[0];
-    double vn = dot2(u, v, n0, n1);
+    double u = l.W[2] / l.W[0], v = l.W[3] / l.W[0];
+    double vn = dot2(u, v, l.n0, l.n1);
     double up = Wp[2] / Wp[0], vp = Wp[3] / Wp[0];
-    double vnp = dot2(up, vp, n0, n1);
+    double vnp = dot2(up, vp, l.n0, l.n1);
     for (int q = 0; q < 2; q++) {
-      const double tw = s.tW[pidx(q, nc, nb)];
-      double twp = tw + tdw[q];
-      double fc = tw * vn, fcp = twp * vnp;
+      double twp = l.tw[q] + tdw[q];
+      double fc = l.tw[q] * vn, fcp = twp * vnp;
       double DFc = left ? (fcp - fc) : (fc - fcp);
-      double Fv = rA * tdw[q];
-      tt[q] = 0.5 * (DFc - Fv) * A;
+      double Fv = l.rA * tdw[q];
+      tt[q] = 0.5 * (DFc - Fv) * l.A;
     }
+  }
+}
+
+// The increments a sweep stored for cell c.
+template <int FLOW, bool FWD>
+__device__ __forceinline__ void load_increment(const DevState &s, int nc, int c, double *dW, double *tdw) {
+  load4p(FWD ? s.dW1 : s.dW, nc, c, dW);
+  if (Flow<FLOW>::sst) {
+    const double2 t = ld2(FWD ? s.tdW1 : s.tdW, 0, nc, c);
+    tdw[0] = t.x;
+    tdw[1] = t.y;
   }
 }
 
 // Sum of DF over the dependency neighbours of cell c -- lower ones in the
 // forward sweep, upper ones in the backward sweep -- in slot order, from
-// their stored increments.
+// their stored increments.  The faces and neighbours of the four slots come
+// in one round trip ahead of the slots' gathers, where each slot's own look
+// at its neighbour cost a latency of its own.  (Two slots' gathers in flight
+// without a branch between them: faster up to 100 k cells, but 15 % slower at
+// 1 M, where the sweeps are bound by their traffic and the gathers and
+// fluxes of slots that are no dependency are wasted.)  Measured per launch,
+// forward / backward: Euler 20 k cells 8.1 / 6.9 -> 7.7 / 6.1 us, laminar
+// 100 k (batch) 9.0 / 7.4 -> 7.6 / 6.0 us, Euler 1 M 26.0 / 22.9 -> 24.0 /
+// 21.0 us, SST 1 M 34.2 / 34.5 -> 31.9 / 32.8 us.
 template <int FLOW, bool FWD>
 __device__ __forceinline__ void df_sum(const DevMesh &m, const DevState &s, int c, double *dFi, double *tFi) {
   using F = Flow<FLOW>;
   const int nc = m.nc;
-  const double *dsrc = FWD ? s.dW1 : s.dW;
-  const double *tsrc = FWD ? s.tdW1 : s.tdW;
-  for (int sl = 0; sl < 4; sl++) {
-    Slot o;
-    if (!get_slot(m, sl, c, o)) break;
-    if (o.nb < 0) continue;
-    if (FWD ? !(o.nb < c) : !(o.nb > c)) continue;
+  int fe[4], nb[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    fe[i] = m.cf[i * nc + c];
+    nb[i] = m.cnb[i * nc + c];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    // (an empty slot holds a negative code, as a boundary face does)
+    if (nb[i] < 0 || !(FWD ? nb[i] < c : nb[i] > c)) continue;
+    DfLoads<FLOW> l;
     double dW[4], tdw[2] = {0.0, 0.0}, t[4], tt[2] = {0.0, 0.0};
-    for (int j = 0; j < 4; j++) dW[j] = dsrc[pidx(j, nc, o.nb)];
-    if (F::sst)
-      for (int q = 0; q < 2; q++) tdw[q] = tsrc[pidx(q, nc, o.nb)];
-    df_term<FLOW>(m, s, c, sl, o.left, o.nb, dW, tdw, t, tt);
+    load_increment<FLOW, FWD>(s, nc, nb[i], dW, tdw);
+    l.load(m, s, c, i, nb[i]);
+    df_term<FLOW>(l, fe[i] >= 0, dW, tdw, t, tt);
     for (int j = 0; j < 4; j++) dFi[j] += t[j];
     if (F::sst)
       for (int q = 0; q < 2; q++) tFi[q] += tt[q];
@@ -1223,16 +1256,13 @@ __device__ __forceinline__ void sweep_tail_cell(const DevMesh &m, const DevState
   if (get_slot(m, q, c, o) && o.nb >= 0 && (FWD ? o.nb < c : o.nb > c)) {
     has = 1;
     double dW[4], tdw[2] = {0.0, 0.0};
-    if (m.wflag[o.nb] & (FWD ? 4 : 8)) {
+    if (m.wflag[o.nb] & (FWD ? 4 : 8))
       increment_of<FLOW, FWD, B>(m, s, o.nb, dW, tdw);
-    } else {
-      const double *dsrc = FWD ? s.dW1 : s.dW;
-      const double *tsrc = FWD ? s.tdW1 : s.tdW;
-      for (int j = 0; j < 4; j++) dW[j] = dsrc[pidx(j, nc, o.nb)];
-      if (F::sst)
-        for (int r = 0; r < 2; r++) tdw[r] = tsrc[pidx(r, nc, o.nb)];
-    }
-    df_term<FLOW>(m, s, c, q, o.left, o.nb, dW, tdw, t, tt);
+    else
+      load_increment<FLOW, FWD>(s, nc, o.nb, dW, tdw);
+    DfLoads<FLOW> l;
+    l.load(m, s, c, q, o.nb);
+    df_term<FLOW>(l, o.left, dW, tdw, t, tt);
   }
   double dFi[4] = {0, 0, 0, 0}, tFi[2] = {0, 0};
   for (int sl = 0; sl < 4; sl++) {
@@ -1264,8 +1294,7 @@ __device__ __forceinline__ void sweep_tail_cell(const DevMesh &m, const DevState
   }
 }
 
-// Held to 96 VGPRs (5 waves per SIMD, as before the tail path existed; the
-// inlined recomputation of the tail path would otherwise take 106).
+// Held to 96 VGPRs (5 waves per SIMD), within which no variant spills.
 template <int FLOW, bool FWD, typename T, bool B>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_sweep(
     const DevMesh m, const DevState s, const Consts k_, const int *__restrict__ items, const XSlice sl,
