@@ -14,6 +14,8 @@
 //   k_sweep   one launch per wave of the forward and the backward sweep; the
 //             backward wave of each cell also writes the updated state into
 //             the second buffer (no separate update pass)
+//   k_levels  the narrow last levels of a sweep that has many (a mesh in its
+//             file's numbering), in one launch
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -790,29 +792,18 @@ __device__ __forceinline__ void carry_state(const DevMesh &m, const DevState &s,
   }
 }
 
-template <int FLOW, typename T, bool B>
-__device__ __forceinline__ void bwd_store(const DevMesh &m, const DevState &s, const Consts &k, int c,
-                                          const double *dW1, const double *tdW1, const double *dFi,
-                                          const double *tFi, double diag) {
+// The update of cell c by its increments: tD divides what is left of the SST
+// increment (tdw = tdW1 - tFi / tD, with tdW1 and tFi given).
+template <int FLOW, typename T>
+__device__ __forceinline__ void bwd_apply(const DevMesh &m, const DevState &s, const Consts &k, int c,
+                                          const double *dW, const double *tdW1, const double *tFi) {
   using F = Flow<FLOW>;
   const int nc = m.nc;
-  if constexpr (B) {
-    // a batch case whose residual failed a check in this iteration keeps
-    // its state (the other cases are independent of it)
-    if (s.err[2 + m.ccase[c]]) {
-      carry_state<FLOW>(m, s, c);
-      return;
-    }
-  }
-  if (frozen_cell(m, c)) {
-    carry_state<FLOW>(m, s, c);
-    return;
-  }
   double W[4], tD[2] = {1.0, 1.0}, tW[2] = {0.0, 0.0}, g5 = 0.0, g6 = 0.0, f2 = 0.0;
   load4p(s.W, nc, c, W);
   if (F::sst) {
     for (int q = 0; q < 2; q++) {
-      tD[q] = s.tD[pidx(q, nc, c)];
+      if (tFi) tD[q] = s.tD[pidx(q, nc, c)];
       tW[q] = s.tW[pidx(q, nc, c)];
     }
     const T *G = pickc<T>(s.grad, s.gradf);
@@ -820,11 +811,8 @@ __device__ __forceinline__ void bwd_store(const DevMesh &m, const DevState &s, c
     g6 = double(G[pidx(6, nc, c)]);
     f2 = double(pickc<T>(s.F2, s.F2f)[c]);
   }
-  double dW[4], Wn[4], Un[4];
-  for (int j = 0; j < 4; j++) {
-    dW[j] = dW1[j] - dFi[j] / diag;
-    Wn[j] = W[j] + dW[j];
-  }
+  double Wn[4], Un[4];
+  for (int j = 0; j < 4; j++) Wn[j] = W[j] + dW[j];
   prim_of(Wn, Un);
   store4p(s.dW, nc, c, dW);
   store4p(s.Wn, nc, c, Wn);
@@ -832,7 +820,7 @@ __device__ __forceinline__ void bwd_store(const DevMesh &m, const DevState &s, c
   if (F::sst) {
     double tdw[2], tw[2];
     for (int q = 0; q < 2; q++) {
-      tdw[q] = tdW1[q] - tFi[q] / tD[q];
+      tdw[q] = tFi ? tdW1[q] - tFi[q] / tD[q] : tdW1[q];
       s.tdW[pidx(q, nc, c)] = tdw[q];
       tw[q] = tW[q] + tdw[q];
     }
@@ -855,6 +843,30 @@ __device__ __forceinline__ void bwd_store(const DevMesh &m, const DevState &s, c
     double h = smax(SST_A1 * tw[1] / rho, f2 * curl);
     s.mutn[c] = SST_A1 * tw[0] / h;
   }
+}
+
+// A cell the backward sweep does not update: an overset hole or receptor
+// cell, or any cell of a batch case whose residual failed a check in this
+// iteration (the other cases are independent of it).
+template <bool B>
+__device__ __forceinline__ bool not_updated(const DevMesh &m, const DevState &s, int c) {
+  if constexpr (B) {
+    if (s.err[2 + m.ccase[c]]) return true;
+  }
+  return frozen_cell(m, c);
+}
+
+template <int FLOW, typename T, bool B>
+__device__ __forceinline__ void bwd_store(const DevMesh &m, const DevState &s, const Consts &k, int c,
+                                          const double *dW1, const double *tdW1, const double *dFi,
+                                          const double *tFi, double diag) {
+  if (not_updated<B>(m, s, c)) {
+    carry_state<FLOW>(m, s, c);
+    return;
+  }
+  double dW[4];
+  for (int j = 0; j < 4; j++) dW[j] = dW1[j] - dFi[j] / diag;
+  bwd_apply<FLOW, T>(m, s, k, c, dW, tdW1, tFi);
 }
 
 // ---------------------------------------------------------------------------
@@ -1335,6 +1347,321 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
   }
 }
 
+// ---------------------------------------------------------------------------
+// Sweeps of many narrow levels.  A mesh in its file's numbering has hundreds
+// of dependency levels per sweep, most of them a few dozen cells: one launch
+// per level then costs a launch's latency per level, whatever the cells.  A
+// sweep's wide first levels keep their launches; its narrow last levels run
+// as one:
+//   k_level_pack    what each of their cells' DF terms reads besides the
+//                   increments (neighbour state, normal, length, r_A;
+//                   residual and diagonal), gathered by the whole chip into
+//                   records in level order
+//   k_levels        one workgroup per case walks the levels with a barrier
+//                   per level (one launch per sweep); it reads the records
+//                   as a stream and a neighbour's increments from a ring of
+//                   the last levels in LDS, or from memory if it is older
+//   k_level_finish  the updated state of their cells, by the whole chip
+// The expressions are the sweep waves', in the same order: the same bits.
+// Measured (LU-SGS iterations, one launch per level before): laminar airfoil,
+// 40 k cells in generator order, 200 levels of about 25 cells per sweep,
+// 1.64 -> 0.33 ms; 400 x 200 quads in row order (599 levels of 200), Euler 7.0
+// -> 1.8 ms; 500 x 400 quads (899 of 400) 12.6 -> 3.8 ms; 20 k-cell Delaunay
+// mesh 0.33 -> 0.21 ms.
+// ---------------------------------------------------------------------------
+// k_levels' threads: kLevelGroups groups, four lanes per cell, one dependency
+// each; chunk i of a case's levels is group i % kLevelGroups' work
+constexpr int kLevelGroups = 4, kLevelCells = 64;  // cells of a chunk
+constexpr int kLevelThreads = kLevelGroups * 4 * kLevelCells;
+// levels whose increments LDS holds: a group's records are loaded while the
+// other groups' chunks, of up to kLevelGroups - 1 levels, are still to come
+constexpr int kLevelRing = kLevelGroups;
+// code of a dependency: LDS ring entry (near) or cell, and flags; -1: none
+constexpr int kCodeNear = 1 << 30, kCodeLeft = 1 << 29, kCodeIndex = (1 << 29) - 1;
+
+// One sweep's narrow levels: positions are their cells by (case, level).
+struct LevelSweep {
+  int n;               // positions
+  const int *pos;      // [nc] position of a cell, -1 if its level is wide
+  const int *cell;     // [n]
+  const int *code;     // [dependencies][n], in slot order
+  const int4 *chunk;   // (first position, cells, ring entry, bit i: a level begins with the i-th chunk from here)
+  const int *coff;     // chunks of each case
+  double *rec;         // [dependencies][pairs][n][2]: (W0,W1) (W2,W3) (nx,ny) (A,r_A) (rho k, rho omega)
+  double *base, *diag; // [n][4], [n]: forward the residual, backward dW1
+  double *tbase, *tdiag;  // SST: [n][2]
+  unsigned char *off;  // bit 0: no increment; bit 1 (forward): no upper neighbour, its dW is dW1
+                       // (bit 2: or 0, not updated)
+};
+struct LevelView {
+  LevelSweep f, b;
+  const int *to_b;     // forward position -> backward position or -1
+};
+
+template <int FLOW>
+__host__ __device__ constexpr int level_pairs() { return FLOW == USG_SST ? 5 : 4; }
+template <int FLOW>
+__host__ __device__ constexpr int level_vars() { return FLOW == USG_SST ? 6 : 4; }
+
+template <int FLOW, bool B>
+__global__ __launch_bounds__(kBlock) void k_level_pack(const DevMesh m, const DevState s, const LevelView v,
+                                                       const NormBlocks nbk) {
+  using F = Flow<FLOW>;
+  if (nbk.kind && (int)blockIdx.x >= nbk.nsweep) {
+    norm_partial_block(m, nbk.R, nbk.b0, nbk.b1, nbk.partial, (int)blockIdx.x - nbk.nsweep);
+    return;
+  }
+  const int c = blockIdx.x * blockDim.x + threadIdx.x, nc = m.nc;
+  if (c >= nc) return;
+  const int pf = v.f.pos[c], pb = v.b.pos[c];
+  if (pf < 0 && pb < 0) return;
+  int nb[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) nb[i] = m.cnb[i * nc + c];
+  const double diag = s.D[c];
+  const int last = m.wflag[c] & 2;
+  const bool fz = frozen_cell(m, c), off = not_updated<B>(m, s, c);
+  // forward: the residual; backward, where a launched level has formed it
+  // already, dW1 (k_levels brings the others)
+  double R[4], dW1[4], tR[2] = {0.0, 0.0}, tdW1[2] = {0.0, 0.0}, tD[2] = {1.0, 1.0};
+  load4p(s.R, nc, c, R);
+  load4p(s.dW1, nc, c, dW1);
+  if (F::sst) {
+    const double2 a = ld2(s.tR, 0, nc, c), b = ld2(s.tD, 0, nc, c), d = ld2(s.tdW1, 0, nc, c);
+    tR[0] = a.x, tR[1] = a.y, tD[0] = b.x, tD[1] = b.y, tdW1[0] = d.x, tdW1[1] = d.y;
+  }
+  auto put = [&](const LevelSweep &w, int pos, int j, const DfLoads<FLOW> &l) {
+    double2 *r = reinterpret_cast<double2 *>(w.rec) + (size_t)j * level_pairs<FLOW>() * w.n + pos;
+    r[0] = make_double2(l.W[0], l.W[1]);
+    r[(size_t)w.n] = make_double2(l.W[2], l.W[3]);
+    r[(size_t)2 * w.n] = make_double2(l.n0, l.n1);
+    r[(size_t)3 * w.n] = make_double2(l.A, l.rA);
+    if (F::sst) r[(size_t)4 * w.n] = make_double2(l.tw[0], l.tw[1]);
+  };
+  int jf = 0, jb = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if (nb[i] < 0) continue;
+    const bool lower = nb[i] < c;
+    if ((lower ? pf : pb) < 0) continue;
+    DfLoads<FLOW> l;
+    l.load(m, s, c, i, nb[i]);
+    if (lower)
+      put(v.f, pf, jf++, l);
+    else
+      put(v.b, pb, jb++, l);
+  }
+  auto head = [&](const LevelSweep &w, int pos, const double *x, const double *tx, int flags) {
+    double2 *o = reinterpret_cast<double2 *>(w.base) + (size_t)2 * pos;
+    o[0] = make_double2(x[0], x[1]);
+    o[1] = make_double2(x[2], x[3]);
+    w.diag[pos] = diag;
+    w.off[pos] = (unsigned char)flags;
+    if (F::sst) {
+      reinterpret_cast<double2 *>(w.tbase)[pos] = make_double2(tx[0], tx[1]);
+      reinterpret_cast<double2 *>(w.tdiag)[pos] = make_double2(tD[0], tD[1]);
+    }
+  };
+  if (pf >= 0) head(v.f, pf, R, tR, (fz ? 1 : 0) | last | (off ? 4 : 0));
+  if (pb >= 0) head(v.b, pb, dW1, tdW1, off ? 1 : 0);
+}
+
+// value of lane K of each group of four lanes
+template <int K>
+__device__ __forceinline__ double quad_lane(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, K * 0x55, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), K * 0x55, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Bound by the latency of one level: barrier, LDS read, flux, four-lane sum,
+// quotient, LDS write.  Everything else is taken out of that chain: the groups
+// take the chunks in turn, and a group between two chunks of its own loads
+// the records of its next one, the codes of the one after that and the place
+// of the third (so nothing is waited for right after it was asked for), and
+// forms the neighbour's flux before the barrier that its chunk waits for.
+// (All threads on every chunk, with three chunks' records in flight: 0.9 us
+// a level instead of 0.55.)
+template <int FLOW, bool FWD>
+__global__ __launch_bounds__(kLevelThreads) void k_levels(const DevState s, const LevelView v, int nc) {
+  using F = Flow<FLOW>;
+  constexpr int kVars = level_vars<FLOW>(), G = kLevelGroups;
+  extern __shared__ __align__(16) double ring[];  // [entries][kVars]
+  const LevelSweep &w = FWD ? v.f : v.b;
+  const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x / (4 * kLevelCells));
+  const int cell = ((int)threadIdx.x >> 2) % kLevelCells, q = (int)threadIdx.x & 3;
+  const double2 *rec = reinterpret_cast<const double2 *>(w.rec);
+  double *dst = FWD ? s.dW1 : s.dW, *tdst = FWD ? s.tdW1 : s.tdW;
+  const int n0 = w.coff[blockIdx.x], n1 = w.coff[blockIdx.x + 1];  // whole rounds of G chunks
+  if (n0 == n1) return;
+  // (the chunk table is not written while this kernel runs: scalar loads)
+  using ConstInt = const __attribute__((address_space(4))) int;
+  const ConstInt *table = (const ConstInt *)(uintptr_t)w.chunk;
+  auto place = [&](int n) {  // what follows a case's last chunk is loaded, never worked on
+    n = min(n, n1);
+    return make_int4(table[4 * n], table[4 * n + 1], table[4 * n + 2], table[4 * n + 3]);
+  };
+
+  // the group's chunk in work or next, its codes ahead, its place ahead
+  int4 ch, ch1, ch2;
+  int code, code1, at = 0, to_b = -1, off = 0;
+  double2 w01, w23, nn, ar, tw, f01, f23, ft;
+  double base = 0.0, diag = 1.0, tbase = 0.0, tdiag = 1.0;
+  double Fc[4], vn = 0.0;
+
+  auto codes = [&](const int4 &p) { return w.code[(size_t)q * w.n + min(p.x + cell, w.n - 1)]; };
+  auto records = [&] {
+    if (cell >= ch.y) return;
+    const int p = ch.x + cell;
+    at = w.cell[p];
+    off = w.off[p];
+    diag = w.diag[p];
+    base = w.base[(size_t)4 * p + q];
+    if (FWD) to_b = v.to_b[p];
+    if (F::sst && q < 2) {
+      tdiag = w.tdiag[(size_t)2 * p + q];
+      tbase = w.tbase[(size_t)2 * p + q];
+    }
+    if (code < 0) return;
+    const double2 *a = rec + (size_t)q * level_pairs<FLOW>() * w.n + p;
+    w01 = a[0];
+    w23 = a[(size_t)w.n];
+    nn = a[(size_t)2 * w.n];
+    ar = a[(size_t)3 * w.n];
+    if (F::sst) tw = a[(size_t)4 * w.n];
+    if (!(code & kCodeNear)) {
+      const int i = code & kCodeIndex;
+      f01 = ld2(dst, 0, nc, i);
+      f23 = ld2(dst, 1, nc, i);
+      if (F::sst) ft = ld2(tdst, 0, nc, i);
+    }
+  };
+  auto next = [&](int n) {  // after the group's chunk n
+    ch = ch1;
+    code = code1;
+    records();
+    ch1 = ch2;
+    code1 = codes(ch1);
+    ch2 = place(n + 3 * G);
+  };
+  // the part of df_term that needs no increment
+  auto flux = [&] {
+    if (cell >= ch.y || code < 0) return;
+    const double W[4] = {w01.x, w01.y, w23.x, w23.y};
+    cons_flux(W, nn.x, nn.y, Fc);
+    if (F::sst) vn = dot2(W[2] / W[0], W[3] / W[0], nn.x, nn.y);
+  };
+  auto work = [&] {
+    if (cell >= ch.y) return;
+    double t[4] = {-0.0, -0.0, -0.0, -0.0}, tt[2] = {-0.0, -0.0};
+    if (code >= 0) {
+      // df_term with Fc (and vn) at hand
+      const bool near = (code & kCodeNear) != 0;
+      const double2 *g = reinterpret_cast<const double2 *>(ring + (near ? code & kCodeIndex : 0) * kVars);
+      double2 a = g[0], b = g[1], e = ft;
+      a.x = near ? a.x : f01.x, a.y = near ? a.y : f01.y;
+      b.x = near ? b.x : f23.x, b.y = near ? b.y : f23.y;
+      if (F::sst) {
+        e = g[2];
+        e.x = near ? e.x : ft.x, e.y = near ? e.y : ft.y;
+      }
+      const bool left = (code & kCodeLeft) != 0;
+      const double dW[4] = {a.x, a.y, b.x, b.y}, Wp[4] = {w01.x + a.x, w01.y + a.y, w23.x + b.x, w23.y + b.y};
+      double Fcp[4];
+      cons_flux(Wp, nn.x, nn.y, Fcp);
+      for (int j = 0; j < 4; j++) {
+        const double DFc = left ? (Fcp[j] - Fc[j]) : (Fc[j] - Fcp[j]);
+        t[j] = 0.5 * (DFc - ar.y * dW[j]) * ar.x;
+      }
+      if (F::sst) {
+        const double vnp = dot2(Wp[2] / Wp[0], Wp[3] / Wp[0], nn.x, nn.y), tdw[2] = {e.x, e.y}, t0[2] = {tw.x, tw.y};
+        for (int r = 0; r < 2; r++) {
+          const double twp = t0[r] + tdw[r], fc = t0[r] * vn, fcp = twp * vnp;
+          const double DFc = left ? (fcp - fc) : (fc - fcp);
+          tt[r] = 0.5 * (DFc - ar.y * tdw[r]) * ar.x;
+        }
+      }
+    }
+    // the four lanes' terms in slot order (an absent one adds -0.0); lane q
+    // keeps component q
+    double sum[4], tsum[2];
+    for (int j = 0; j < 4; j++) {
+      sum[j] = 0.0 + quad_lane<0>(t[j]);
+      sum[j] += quad_lane<1>(t[j]);
+      sum[j] += quad_lane<2>(t[j]);
+      sum[j] += quad_lane<3>(t[j]);
+    }
+    if (F::sst)
+      for (int j = 0; j < 2; j++) {
+        tsum[j] = 0.0 + quad_lane<0>(tt[j]);
+        tsum[j] += quad_lane<1>(tt[j]);
+        tsum[j] += quad_lane<2>(tt[j]);
+        tsum[j] += quad_lane<3>(tt[j]);
+      }
+    const double dF = q == 0 ? sum[0] : q == 1 ? sum[1] : q == 2 ? sum[2] : sum[3];
+    double dW = FWD ? (-base - dF) / diag : base - dF / diag;
+    if (off & 1) dW = 0.0;
+    double *e = ring + (size_t)(ch.z + cell) * kVars;
+    e[q] = dW;
+    dst[pidx(q, nc, at)] = dW;
+    if (FWD && to_b >= 0) v.b.base[(size_t)4 * to_b + q] = dW;
+    if (FWD && (off & 2)) s.dW[pidx(q, nc, at)] = off & 4 ? 0.0 : dW;
+    if (F::sst && q < 2) {
+      const double tF = q == 0 ? tsum[0] : tsum[1];
+      double td = FWD ? (-tbase - tF) / tdiag : tbase - tF / tdiag;
+      if (off & 1) td = 0.0;
+      e[4 + q] = td;
+      tdst[pidx(q, nc, at)] = td;
+      if (FWD && to_b >= 0) v.b.tbase[(size_t)2 * to_b + q] = td;
+      if (FWD && (off & 2)) s.tdW[pidx(q, nc, at)] = off & 4 ? 0.0 : td;
+    }
+  };
+
+  int n = n0 + group;
+  ch = place(n);
+  code = codes(ch);
+  records();
+  ch1 = place(n + G);
+  code1 = codes(ch1);
+  ch2 = place(n + 2 * G);
+  const int before = place(n0).w;  // the levels that begin with the other groups' first chunks
+  for (int i = 0; i < group; i++)
+    if (before >> i & 1) __syncthreads();
+  for (; n < n1; n += G) {
+    const int begins = ch.w;
+    flux();
+    if (begins & 1) __syncthreads();
+    work();
+    if (begins & 2) __syncthreads();
+    next(n);
+#pragma unroll
+    for (int i = 2; i < G; i++)
+      if (begins >> i & 1) __syncthreads();
+  }
+}
+
+// The updated state of the cells whose dW k_levels formed.
+template <int FLOW, typename T, bool B>
+__global__ __launch_bounds__(kBlock) void k_level_finish(const DevMesh m, const DevState s, const Consts k_,
+                                                         const LevelView v, const NormBlocks nbk) {
+  if (nbk.kind && (int)blockIdx.x >= nbk.nsweep) {
+    norm_ring_block(nbk.partial, nbk.boff, nbk.ring, nbk.cap, nbk.ctr, 0, 1);
+    return;
+  }
+  const int c = blockIdx.x * blockDim.x + threadIdx.x, nc = m.nc;
+  if (c >= nc) return;
+  if (v.b.pos[c] < 0 && !((m.wflag[c] & 2) && v.f.pos[c] >= 0)) return;
+  if (not_updated<B>(m, s, c)) {
+    carry_state<FLOW>(m, s, c);
+    return;
+  }
+  const Consts k = case_consts<B>(m, k_, c);
+  double dW[4], tdW[2] = {0.0, 0.0};
+  load_increment<FLOW, false>(s, nc, c, dW, tdW);
+  bwd_apply<FLOW, T>(m, s, k, c, dW, tdW, nullptr);
+}
+
 // RK5 stage (RungeKuttaStrategy.h:39-72): W_now = W0 + alpha*dt*(-R)/V ; U = prim(W_now)
 __global__ __launch_bounds__(kBlock) void k_rk_stage(const DevMesh m, const DevState s, double cfl, double alpha,
                                                      int stage, int visc_sst) {
@@ -1757,6 +2084,11 @@ struct usg_ctx {
   // that are contiguous cell ranges (the colour-blocked numbering), whose
   // parts are then contiguous sub-ranges
   bool face_ident = false, sweep_ident = false;
+  // sweeps of many narrow levels (k_levels): the view, and the LDS ring
+  bool levels = false;
+  LevelView lv{};
+  size_t level_lds = 0;
+  int level_from[2] = {0, 0};  // first level of the forward / backward sweep in k_levels
   int tile_bs = 0, tile_stride = 0;
   int *d_tfoff = nullptr, *d_tface = nullptr;
   unsigned short *d_lfs = nullptr;
@@ -1995,11 +2327,207 @@ static int sweep_launches(const usg_ctx *c) {
   return std::max(0, nfw - 1 - (c->fwd_tail ? 1 : 0)) + std::max(0, nbw - 1 - (c->bwd_tail ? 1 : 0));
 }
 
+// A sweep launch takes 3.5-6 us however few cells it holds, a level of up to
+// kLevelGroups * kLevelCells cells in k_levels a tenth of that, so the narrow last levels of
+// the two sweeps go to k_levels when that replaces at least kLevelMin
+// launches (which repay its own four).  A level is narrow up to kLevelWidth
+// cells of a case: two rounds of chunks, where the launch is about as fast.
+constexpr int kLevelMin = 12, kLevelWidth = 8 * kLevelCells;
+
+template <int FLOW>
+static bool level_lds_limit(size_t bytes) {
+  for (const void *f : {reinterpret_cast<const void *>(&k_levels<FLOW, true>),
+                        reinterpret_cast<const void *>(&k_levels<FLOW, false>)})
+    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+  return true;
+}
+
+// The narrow last levels of one sweep: level of every cell, first narrow
+// level, and the narrow cells by (case, level).
+struct LevelOrder {
+  std::vector<int> level, pos, order, first;  // first[case]: first position
+  int nw = 0, from = 0, width = 1;            // width: cells of the widest narrow level of a case
+};
+
+static LevelOrder order_levels(const usg_ctx *c, bool fwd) {
+  const HostMesh &h = c->hm;
+  const int nc = h.nc;
+  const std::vector<int> &list = fwd ? h.fwd_list : h.bwd_list, &poff = fwd ? h.fwd_poff : h.bwd_poff;
+  LevelOrder o;
+  o.nw = (int)poff.size() / (kXcd + 1);
+  o.level.assign(nc, 0);
+  for (int w = 0; w < o.nw; w++)
+    for (int i = poff[(size_t)w * (kXcd + 1)]; i < poff[(size_t)w * (kXcd + 1) + kXcd]; i++) o.level[list[i]] = w;
+  std::vector<std::vector<int>> cnt(c->ncase, std::vector<int>(o.nw, 0));
+  o.from = 1;  // level 0 runs in k_cell and the forward launches
+  for (int k = 0; k < c->ncase; k++) {
+    for (int i = h.case_cell[k]; i < h.case_cell[k + 1]; i++) cnt[k][o.level[i]]++;
+    for (int w = 1; w < o.nw; w++)
+      if (cnt[k][w] > kLevelWidth) o.from = std::max(o.from, w + 1);
+  }
+  o.pos.assign(nc, -1);
+  o.first.assign(1, 0);
+  std::vector<int> at(o.nw);
+  for (int k = 0; k < c->ncase; k++) {
+    int p = o.first[k];
+    for (int w = o.from; w < o.nw; w++) {
+      at[w] = p;
+      p += cnt[k][w];
+      o.width = std::max(o.width, cnt[k][w]);
+    }
+    o.order.resize(p);
+    for (int i = h.case_cell[k]; i < h.case_cell[k + 1]; i++)
+      if (o.level[i] >= o.from) {
+        o.pos[i] = at[o.level[i]]++;
+        o.order[o.pos[i]] = i;
+      }
+    o.first.push_back(p);
+  }
+  return o;
+}
+
+// Chunks and dependency codes of one sweep's narrow levels, uploaded with its
+// record buffers.  A chunk's records are loaded after the barrier of the
+// chunk kLevelGroups - 1 before it, when the increments of all levels before
+// that one's are in memory: a neighbour kLevelRing or more levels back is
+// read from there, a nearer one from the ring, whose entries are overwritten
+// kLevelRing levels after their own.
+static int upload_levels(usg_ctx *c, bool fwd, const LevelOrder &o, LevelSweep &v) {
+  const HostMesh &h = c->hm;
+  const int n = (int)o.order.size();
+  std::vector<int> start(n, 0), coff(1, 0), code(4 * (size_t)n, -1);  // start: first position of the level
+  std::vector<int4> chunk;
+  for (int k = 0; k < c->ncase; k++) {
+    for (int p = o.first[k]; p < o.first[k + 1];) {
+      const int l = o.level[o.order[p]];
+      int e = p;
+      while (e < o.first[k + 1] && o.level[o.order[e]] == l) start[e++] = p;
+      for (int a = p; a < e; a += kLevelCells)
+        chunk.push_back(
+            make_int4(a, std::min(kLevelCells, e - a), (l % kLevelRing) * o.width + (a - p), a == p ? 1 : 0));
+      p = e;
+    }
+    // whole rounds of kLevelGroups chunks
+    while (chunk.size() % kLevelGroups) chunk.push_back(make_int4(0, 0, 0, 0));
+    for (int j = coff.back(); j < (int)chunk.size(); j++)
+      for (int i = 1; i < kLevelGroups && j + i < (int)chunk.size(); i++) chunk[j].w |= (chunk[j + i].w & 1) << i;
+    coff.push_back((int)chunk.size());
+  }
+  chunk.push_back(make_int4(0, 0, 0, 0));  // what the last case loads ahead of its end
+  int ndep = 1;
+  for (int p = 0; p < n; p++) {
+    const int i = o.order[p];
+    int j = 0;
+    for (int sl = 0; sl < h.cnf[i]; sl++) {
+      const int f = h.cface[4 * i + sl];
+      const bool left = h.flc[f] == i;
+      const int nb = left ? h.frc[f] : h.flc[f];
+      if (nb < 0 || (fwd ? nb > i : nb < i)) continue;
+      const int l = o.level[nb], flag = left ? kCodeLeft : 0;
+      const bool near = l >= o.from && o.level[i] - l < kLevelRing;
+      code[(size_t)(j++) * n + p] =
+          near ? flag | kCodeNear | ((l % kLevelRing) * o.width + (o.pos[nb] - start[o.pos[nb]])) : flag | nb;
+    }
+    ndep = std::max(ndep, j);
+  }
+  const bool sst = c->prm.flow == USG_SST;
+  const size_t N = n, pairs = sst ? 5 : 4;
+  int rc = USG_OK;
+  v.n = n;
+  if ((rc = upload(c, const_cast<int **>(&v.pos), o.pos.data(), o.pos.size())) ||
+      (rc = upload(c, const_cast<int **>(&v.cell), o.order.data(), N)) ||
+      (rc = upload(c, const_cast<int **>(&v.code), code.data(), 4 * N)) ||
+      (rc = upload(c, const_cast<int4 **>(&v.chunk), chunk.data(), chunk.size())) ||
+      (rc = upload(c, const_cast<int **>(&v.coff), coff.data(), coff.size())) ||
+      (rc = dalloc(c, &v.rec, ndep * pairs * N * 2)) || (rc = dalloc(c, &v.base, 4 * N)) ||
+      (rc = dalloc(c, &v.diag, N)) || (rc = dalloc(c, &v.off, N)))
+    return rc;
+  if (sst && ((rc = dalloc(c, &v.tbase, 2 * N)) || (rc = dalloc(c, &v.tdiag, 2 * N)))) return rc;
+  HIPCHK(hipStreamSynchronize(c->stream));  // the host arrays go
+  return USG_OK;
+}
+
+static int build_levels(usg_ctx *c) {
+  const HostMesh &h = c->hm;
+  if ((int)(h.fwd_poff.size() + h.bwd_poff.size()) / (kXcd + 1) - 2 < kLevelMin) return USG_OK;
+  const LevelOrder f = order_levels(c, true), b = order_levels(c, false);
+  if (f.nw - f.from + b.nw - b.from < kLevelMin) return USG_OK;
+  int dev = 0, limit = 0;
+  HIPCHK(hipGetDevice(&dev));
+  HIPCHK(hipDeviceGetAttribute(&limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  const size_t lds = (size_t)kLevelRing * std::max(f.width, b.width) * sizeof(double) *
+                     (c->prm.flow == USG_SST ? level_vars<USG_SST>() : level_vars<USG_EULER>());
+  if (lds > (size_t)limit) return USG_OK;
+  const bool ok = c->prm.flow == USG_EULER     ? level_lds_limit<USG_EULER>(lds)
+                  : c->prm.flow == USG_LAMINAR ? level_lds_limit<USG_LAMINAR>(lds)
+                                               : level_lds_limit<USG_SST>(lds);
+  if (!ok) {
+    (void)hipGetLastError();  // the sweeps keep their launches
+    return USG_OK;
+  }
+  std::vector<int> to_b(f.order.size());
+  for (size_t p = 0; p < to_b.size(); p++) to_b[p] = b.pos[f.order[p]];
+  int rc = USG_OK;
+  if ((rc = upload_levels(c, true, f, c->lv.f)) || (rc = upload_levels(c, false, b, c->lv.b)) ||
+      (rc = upload(c, const_cast<int **>(&c->lv.to_b), to_b.data(), to_b.size())))
+    return rc;
+  HIPCHK(hipStreamSynchronize(c->stream));
+  c->level_lds = lds;
+  c->level_from[0] = f.from;
+  c->level_from[1] = b.from;
+  c->levels = true;
+  return USG_OK;
+}
+
+// Wave w of a sweep as a launch of its own.
+template <int FLOW, bool FWD, typename T, bool B>
+static void launch_wave(usg_ctx *c, int w, const NormBlocks &nb, int extra, const SweepTail &tl) {
+  const HostMesh &h = c->hm;
+  const int bs = c->blk[USG_K_SWEEP];
+  const XSlice sl = slice(&(FWD ? h.fwd_poff : h.bwd_poff)[(size_t)w * (kXcd + 1)]);
+  hipLaunchKernelGGL((k_sweep<FLOW, FWD, T, B>), dim3(xgrid(sl, bs) + tl.nblk + extra), dim3(bs), 0, c->stream, c->dm,
+                     c->ds, c->k, c->sweep_ident ? nullptr : FWD ? c->d_fwd : c->d_bwd, sl, nb, tl);
+}
+
+// Both sweeps with their narrow levels in k_levels.
+template <int FLOW, typename T, bool B>
+static void launch_level_sweeps(usg_ctx *c, bool fuse_norm) {
+  NormBlocks none, nb, nb2;
+  if (fuse_norm) {
+    nb.kind = 1;
+    nb.nsweep = c->nblk;
+    nb.cap = kRing;
+    nb.R = c->ds.R;
+    nb.b0 = c->d_nb0;
+    nb.b1 = c->d_nb1;
+    nb.boff = c->d_nboff;
+    nb.partial = c->d_partial;
+    nb.ring = c->d_ring;
+    nb.ctr = c->d_ctr;
+    nb2 = nb;
+    nb2.kind = 2;
+  }
+  for (int w = 1; w < c->level_from[0]; w++) launch_wave<FLOW, true, T, B>(c, w, none, 0, SweepTail{});
+  hipLaunchKernelGGL((k_level_pack<FLOW, B>), dim3(c->nblk + (fuse_norm ? c->nnb : 0)), dim3(kBlock), 0, c->stream,
+                     c->dm, c->ds, c->lv, nb);
+  hipLaunchKernelGGL((k_levels<FLOW, true>), dim3(c->ncase), dim3(kLevelThreads), c->level_lds, c->stream, c->ds,
+                     c->lv, c->hm.nc);
+  for (int w = 1; w < c->level_from[1]; w++) launch_wave<FLOW, false, T, B>(c, w, none, 0, SweepTail{});
+  hipLaunchKernelGGL((k_levels<FLOW, false>), dim3(c->ncase), dim3(kLevelThreads), c->level_lds, c->stream, c->ds,
+                     c->lv, c->hm.nc);
+  hipLaunchKernelGGL((k_level_finish<FLOW, T, B>), dim3(c->nblk + (fuse_norm ? 1 : 0)), dim3(kBlock), 0, c->stream,
+                     c->dm, c->ds, c->k, c->lv, nb2);
+}
+
 // With fuse_norm, the first two sweep launches of the iteration also carry
 // the residual norm into the ring (NormBlocks): the partial sums on the
 // first, the ring sum on the second (forward or backward: neither writes R).
 template <int FLOW, typename T, bool B>
 static void launch_sweeps(usg_ctx *c, bool fuse_norm) {
+  if (c->levels) {
+    launch_level_sweeps<FLOW, T, B>(c, fuse_norm);
+    return;
+  }
   const HostMesh &h = c->hm;
   const int bs = c->blk[USG_K_SWEEP];
   int launch = 0;
@@ -2026,25 +2554,17 @@ static void launch_sweeps(usg_ctx *c, bool fuse_norm) {
   // a small last wave runs as a tail of the wave before it
   const int nw = (int)h.fwd_poff.size() / (kXcd + 1);
   for (int w = 1; w < nw - (c->fwd_tail ? 1 : 0); w++) {
-    XSlice sl = slice(&h.fwd_poff[(size_t)w * (kXcd + 1)]);
-    const int nmain = xgrid(sl, bs);
     const SweepTail tl = c->fwd_tail && w == nw - 2 ? tail_of(h.fwd_poff, bs) : SweepTail{};
-    const int ntail = tl.nblk;
     int extra = 0;
-    const NormBlocks nb = norm_blocks(nmain + ntail, extra);
-    hipLaunchKernelGGL((k_sweep<FLOW, true, T, B>), dim3(nmain + ntail + extra), dim3(bs), 0, c->stream, c->dm,
-                       c->ds, c->k, c->sweep_ident ? nullptr : c->d_fwd, sl, nb, tl);
+    const NormBlocks nb = norm_blocks(xgrid(slice(&h.fwd_poff[(size_t)w * (kXcd + 1)]), bs) + tl.nblk, extra);
+    launch_wave<FLOW, true, T, B>(c, w, nb, extra, tl);
   }
   const int nbw = (int)h.bwd_poff.size() / (kXcd + 1);
   for (int w = 1; w < nbw - (c->bwd_tail ? 1 : 0); w++) {
-    XSlice sl = slice(&h.bwd_poff[(size_t)w * (kXcd + 1)]);
-    const int nmain = xgrid(sl, bs);
     const SweepTail tl = c->bwd_tail && w == nbw - 2 ? tail_of(h.bwd_poff, bs) : SweepTail{};
-    const int ntail = tl.nblk;
     int extra = 0;
-    const NormBlocks nb = norm_blocks(nmain + ntail, extra);
-    hipLaunchKernelGGL((k_sweep<FLOW, false, T, B>), dim3(nmain + ntail + extra), dim3(bs), 0, c->stream, c->dm,
-                       c->ds, c->k, c->sweep_ident ? nullptr : c->d_bwd, sl, nb, tl);
+    const NormBlocks nb = norm_blocks(xgrid(slice(&h.bwd_poff[(size_t)w * (kXcd + 1)]), bs) + tl.nblk, extra);
+    launch_wave<FLOW, false, T, B>(c, w, nb, extra, tl);
   }
 }
 
@@ -2469,6 +2989,7 @@ static int ctx_setup(usg_ctx *c, usg_ctx **out) {
   CK(ensure_norms(c, 16 * c->ncase));
   CK(dalloc(c, &c->d_ring, (size_t)kRing * c->ncase));
   CK(dalloc(c, &c->d_ctr, 1));
+  CK(build_levels(c));
 #undef CK
   if (hipStreamSynchronize(c->stream) != hipSuccess) {
     usg_ctx_destroy(c);
@@ -2599,7 +3120,7 @@ static void launch_norm_ring(usg_ctx *c) {
 // The norm rides on the sweep launches for a single case whose sweeps use
 // kBlock-thread blocks and make at least two launches.
 static bool fuse_norm(const usg_ctx *c) {
-  return c->ncase == 1 && c->blk[USG_K_SWEEP] == kBlock && sweep_launches(c) >= 2;
+  return c->ncase == 1 && (c->levels || (c->blk[USG_K_SWEEP] == kBlock && sweep_launches(c) >= 2));
 }
 
 // One LU-SGS iteration (LUSGSIntegrator::UpdateSerial): residual, norm into
