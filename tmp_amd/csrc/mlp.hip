@@ -7,10 +7,13 @@
 //   B (32 x 16): column l % 16, k = 8 * (l / 16) .. +7
 //   C (16 x 16): column l % 16, rows 4 * (l / 16) .. +3  (4 floats)
 // (checked against the CPU by usg_mlp_mfma_check).  Activations are kept
-// twice: row-major [P][K] (the A operand of the forward and data-gradient
-// products, 8 consecutive k per lane) and point-blocked [P/8][K][8] (both
-// operands of the weight-gradient product, which reduces over points: 8
-// consecutive points per lane).  Every operand load is one 16-byte load.
+// twice: as rows in LDS (the A operand of the forward and data-gradient
+// products, 8 consecutive k per lane) and in memory as operands of the
+// weight-gradient product, which reduces over points (8 consecutive points per
+// lane).  Every operand load is one 16-byte load.
+//
+// A training step is two launches: k_net (batch assembly, forward pass, loss,
+// data gradients) and k_weights (weight and bias gradients, Adam).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -60,248 +63,488 @@ __device__ __forceinline__ float sigmoid(float z) { return 1.0f / (1.0f + expf(-
 __device__ __forceinline__ bf16x8 load8(const bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
 // ---------------------------------------------------------------------------
-// Forward of one layer: Z = X W + b over 64 points x NT*16 outputs per block
-// (4 waves x 16 points).  Wt is W transposed ([N][K]) so that the B operand
-// is 8 consecutive k of one output.  ACT: H = bf16(silu(Z)) row-major (and
-// point-blocked + Z kept when TRAIN); else Z is the network output.
+// The network as the kernels see it.  Weights come as MFMA operands: `wf` the
+// B fragments of the forward product (reduction over k), `wb` those of the
+// data gradient (reduction over n), each fragment 64 lanes x 8 values in lane
+// order, so that a wave loads one with a single contiguous kilobyte.  Layers
+// follow one another in every array; where a layer begins is arithmetic on
+// the shape (a table would put a dependent load before each layer).
 // ---------------------------------------------------------------------------
-template <int NT, bool ACT, bool TRAIN>
-__global__ __launch_bounds__(256) void k_fwd(const bf16 *__restrict__ X, int K, const bf16 *__restrict__ Wt,
-                                             const float *__restrict__ b, int N, float *__restrict__ Z,
-                                             bf16 *__restrict__ H, bf16 *__restrict__ Hb) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int p0 = blockIdx.x * 64 + wave * 16;
-  const int n0 = blockIdx.y * NT * 16;
-  floatx4 acc[NT];
-  for (int t = 0; t < NT; t++) acc[t] = floatx4{0, 0, 0, 0};
-  const bf16 *xa = X + (size_t)(p0 + lane % 16) * K + (lane / 16) * 8;
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    const bf16x8 a = load8(xa + k0);
-    for (int t = 0; t < NT; t++) {
-      const bf16x8 bv = load8(Wt + (size_t)(n0 + t * 16 + lane % 16) * K + k0 + (lane / 16) * 8);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[t], 0, 0, 0);
-    }
-  }
-  for (int t = 0; t < NT; t++) {
-    const int n = n0 + t * 16 + lane % 16;
-    for (int r = 0; r < 4; r++) {
-      const int p = p0 + (lane / 16) * 4 + r;
-      const float z = acc[t][r] + b[n];
-      if (!ACT) {
-        Z[(size_t)p * N + n] = z;
-        continue;
-      }
-      if (TRAIN) Z[(size_t)p * N + n] = z;
-      const bf16 h = to_bf16(z * sigmoid(z));
-      H[(size_t)p * N + n] = h;
-      if (TRAIN) Hb[((size_t)(p / 8) * N + n) * 8 + p % 8] = h;
+constexpr int kOut = 32;   // padded outputs of the last layer
+struct Net {
+  int nl, W, K0, nin, nout;  // layers, width, padded and real inputs, outputs
+  long P;                    // points (training; a multiple of 128)
+  bf16 *wf, *wb;
+  bf16 *in;                  // input of each layer, P x K (pt_index; training)
+  bf16 *dz;                  // output gradient of each layer, P x N (pt_index; training)
+  bf16 *h;                   // rows of each hidden output [P][W] that LDS cannot hold (training)
+  float *w, *b;              // FP32 masters, compact
+  __host__ __device__ int K(int l) const { return l == 0 ? K0 : W; }
+  __host__ __device__ int N(int l) const { return l == nl - 1 ? kOut : W; }
+  __host__ __device__ int k(int l) const { return l == 0 ? nin : W; }
+  __host__ __device__ int n(int l) const { return l == nl - 1 ? nout : W; }
+  __host__ __device__ long frag(int l) const { return l == 0 ? 0 : (long)K0 * W + (long)(l - 1) * W * W; }
+  __host__ __device__ long inp(int l) const { return l == 0 ? 0 : P * K0 + (l - 1) * P * W; }
+  __host__ __device__ long out(int l) const { return l * P * W; }
+  __host__ __device__ long ow(int l) const { return l == 0 ? 0 : (long)nin * W + (long)(l - 1) * W * W; }
+  __host__ __device__ long ob(int l) const { return (long)l * W; }
+};
+__host__ __device__ __forceinline__ size_t wf_index(int k, int n, int N) {
+  return ((size_t)((k / 32) * (N / 16) + n / 16) * 64 + (k % 32) / 8 * 16 + n % 16) * 8 + k % 8;
+}
+__host__ __device__ __forceinline__ size_t wb_index(int k, int n, int K) {
+  return ((size_t)((n / 32) * (K / 16) + k / 16) * 64 + (n % 32) / 8 * 16 + k % 16) * 8 + n % 8;
+}
+
+// Inputs and output gradients for the weight gradient, in MFMA operand order
+// too: the fragment of points 32 q .. 32 q + 31 and columns 16 c .. 16 c + 15
+// (width N) is the kilobyte q * N / 16 + c, its lanes 16 columns of each
+// 8-point block in turn.  (8-point blocks of all columns, whose quarters of a
+// fragment lie 4 KB apart, met in the same few L2 channels.)
+__host__ __device__ __forceinline__ size_t pt_index(long p, int n, int N) {
+  return ((size_t)(p / 32) * (N / 16) + n / 16) * 512 + ((p % 32) / 8 * 16 + n % 16) * 8 + p % 8;
+}
+
+// Where a pass takes its points from: rows idx[0..nv) of the resident set
+// (bf16 inputs padded to K0, fp32 targets), or nv rows of x and y as the
+// caller gave them.
+struct Points {
+  const bf16 *xs;
+  const float *ys;
+  const int *idx;
+  const float *x;
+  const float *y;
+  int nv;
+};
+
+// exp by extended-precision reduction (Cody and Waite): x log2(e) as a rounded
+// product and its remainder, 2^n times 2^f with |f| <= 1/2.  |x| <= 87, where
+// neither end of the range is near.
+__device__ __forceinline__ float exp_mid(float x) {
+  const float c = 1.44269504088896340736f, c2 = (float)(1.44269504088896340736 - (double)c);
+  const float t = x * c;
+  const float lo = __builtin_fmaf(x, c2, __builtin_fmaf(x, c, -t));
+  const float n = __builtin_rintf(t);
+  return __builtin_ldexpf(__builtin_amdgcn_exp2f((t - n) + lo), (int)n);
+}
+// 1 / x, correctly rounded for 1 <= x < 2^126: two Newton steps on the
+// approximate reciprocal, the second on the quotient's remainder (equal to the
+// quotient for every such x).  No operand needs the scaling of a general
+// division.
+__device__ __forceinline__ float recip_mid(float x) {
+  float r = __builtin_amdgcn_rcpf(x);
+  r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+// sigmoid of four values: 16 instructions each where |z| <= 87, against 24 of
+// expf and a division, which take the rest
+__device__ __forceinline__ void sigmoid4(const float (&z)[4], float (&s)[4]) {
+  if (fmaxf(fmaxf(fabsf(z[0]), fabsf(z[1])), fmaxf(fabsf(z[2]), fabsf(z[3]))) <= 87.0f)
+    for (int r = 0; r < 4; r++) s[r] = recip_mid(1.0f + exp_mid(-z[r]));
+  else
+    for (int r = 0; r < 4; r++) s[r] = sigmoid(z[r]);
+}
+typedef bf16 bf16x4u __attribute__((ext_vector_type(4)));
+// four FP32 -> BF16, round to nearest even (as to_bf16)
+__device__ __forceinline__ bf16x4u to_bf16x4(const float (&f)[4]) {
+  typedef float floatx2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const uint32_t a = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{f[0], f[1]}), bf16x2));
+  const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2{f[2], f[3]}), bf16x2));
+  return bf16x4u{(bf16)a, (bf16)(a >> 16), (bf16)b, (bf16)(b >> 16)};
+}
+
+constexpr int kTile = 32;  // points per block of k_net
+constexpr int kPad = 8;    // bf16 added to a row in LDS: 16 rows then start in different banks
+
+// The B fragments of two n tiles of a product of `steps` k steps (a shorter
+// one loads its last step again).  No branch: a load in a branch would make
+// every later wait one for all loads.
+template <int T>
+__device__ __forceinline__ void load_frags(bf16x8 *b, const bf16 *w, int steps, int tiles, int tile) {
+  const int lane = threadIdx.x % kWave;
+#pragma unroll
+  for (int s = 0; s < T; s++)
+    for (int t = 0; t < 2; t++)
+      b[2 * s + t] = load8(w + ((size_t)(min(s, steps - 1) * tiles + tile + t) * 64 + lane) * 8);
+}
+
+// acc[p tile][n tile] of one wave: 32 points x 32 outputs, A rows in LDS
+template <int T>
+__device__ __forceinline__ void product(floatx4 (&acc)[2][2], const bf16 *a, int lda, const bf16x8 *b, int steps) {
+  const int lane = threadIdx.x % kWave;
+  for (int i = 0; i < 2; i++)
+    for (int t = 0; t < 2; t++) acc[i][t] = floatx4{0, 0, 0, 0};
+  const bf16 *r = a + (lane % 16) * lda + (lane / 16) * 8;
+#pragma unroll
+  for (int s = 0; s < T; s++) {
+    if (s >= steps) continue;
+    const bf16x8 a0 = load8(r + s * 32), a1 = load8(r + 16 * lda + s * 32);
+    for (int t = 0; t < 2; t++) {
+      acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[2 * s + t], acc[0][t], 0, 0, 0);
+      acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[2 * s + t], acc[1][t], 0, 0, 0);
     }
   }
 }
 
-// ---------------------------------------------------------------------------
-// Data gradient through one layer: dH = dZ W^T (reduction over its N
-// outputs), then dZ_prev = bf16(dH * silu'(Z_prev)) row-major and
-// point-blocked.  W is [K][N] so that the B operand is 8 consecutive n of
-// one input k.
-// ---------------------------------------------------------------------------
-template <int NT>
-__global__ __launch_bounds__(256) void k_bwd_data(const bf16 *__restrict__ dZ, int N, const bf16 *__restrict__ W,
-                                                  int K, const float *__restrict__ Zp, bf16 *__restrict__ dZp,
-                                                  bf16 *__restrict__ dZpb) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int p0 = blockIdx.x * 64 + wave * 16;
-  const int k0 = blockIdx.y * NT * 16;
-  floatx4 acc[NT];
-  for (int t = 0; t < NT; t++) acc[t] = floatx4{0, 0, 0, 0};
-  const bf16 *da = dZ + (size_t)(p0 + lane % 16) * N + (lane / 16) * 8;
-  for (int n0 = 0; n0 < N; n0 += 32) {
-    const bf16x8 a = load8(da + n0);
-    for (int t = 0; t < NT; t++) {
-      const bf16x8 bv = load8(W + (size_t)(k0 + t * 16 + lane % 16) * N + n0 + (lane / 16) * 8);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[t], 0, 0, 0);
-    }
-  }
-  for (int t = 0; t < NT; t++) {
-    const int k = k0 + t * 16 + lane % 16;
-    for (int r = 0; r < 4; r++) {
-      const int p = p0 + (lane / 16) * 4 + r;
-      const float z = Zp[(size_t)p * K + k];
-      const float s = sigmoid(z);
-      const bf16 d = to_bf16(acc[t][r] * (s * (1.0f + z * (1.0f - s))));
-      dZp[(size_t)p * K + k] = d;
-      dZpb[((size_t)(p / 8) * K + k) * 8 + p % 8] = d;
-    }
-  }
+// Four values of one column n for points p, p+1, p+2, p+3 of the block (p a
+// multiple of 4): into rows in LDS, and into the operand of the weight gradient.
+__device__ __forceinline__ void put4(bf16 *rows, int ld, bf16 *op, int p0, int N, int p, int n,
+                                     bf16x4u v) {
+  for (int r = 0; r < 4; r++) rows[(p + r) * ld + n] = v[r];
+  if (op) *reinterpret_cast<bf16x4u *>(op + pt_index(p0, 0, N) + pt_index(p, n, N)) = v;
 }
 
 // ---------------------------------------------------------------------------
-// Row-major product with the B tile in LDS: C[P][N] = A[P][K] x B, B given
-// transposed (Bt[N][K]).  A block (4 waves) owns 128 points x 64 outputs;
-// each wave 32 points x 64 outputs (2 x 4 MFMA tiles per k step).  The
-// block's 64 rows of Bt are staged in LDS once (rows padded by 8 bf16 so
-// that the 16 lanes reading one column group hit different banks).
-// EPI 0: forward, Z = C + b, H = bf16(silu(Z)) (+ blocked copy and Z when
-// TRAIN); EPI 1: data gradient, dZp = bf16(C * silu'(Zp)) row-major and
-// blocked.
+// k_net: the whole network on kTile points per block.
+//   PREDICT: the outputs of every point.
+//   TRAIN: the forward pass, the loss and the data gradients back to the first
+//   layer; the inputs and output gradients of every layer go to memory as
+//   operands of k_weights.
+// W is the width; W / 32 waves, each 32 outputs of a layer.  Activations stay
+// in LDS as rows, all layers' in training (118 KB at 8 x 256; a deeper
+// network's lower layers go through memory): the backward pass forms each
+// pre-activation again from them, with the forward pass's own product, which
+// costs a third more matrix work but no 4-byte value per activation to memory
+// and back.  A layer's weights come from L2 into registers while the previous
+// layer's activation is in work.
+// Bound by the SiLU and its derivative: a layer's forward activation takes
+// about 4500 of its 5750 cycles, the derivative 6600 of 8900; products and
+// barriers the rest, and the first loads of the points 12000 of a block's
+// 120000 cycles.  Measured at 8 x 256 on 16384 points: 112 us, against 350 us
+// for a launch per product (and one each for the batch, the loss and the last
+// layer); inference of 12576 points 50 us against 98 us.
 // ---------------------------------------------------------------------------
-constexpr int kBN = 64;    // outputs per block
-constexpr int kBP = 128;   // points per block
-template <int EPI, bool TRAIN>
-__global__ __launch_bounds__(256) void k_gemm(const bf16 *__restrict__ A, int K, const bf16 *__restrict__ Bt,
-                                              const float *__restrict__ bias, int N, const float *__restrict__ Zp,
-                                              float *__restrict__ Z, bf16 *__restrict__ H, bf16 *__restrict__ Hb) {
-  extern __shared__ __align__(16) bf16 sB[];  // [kBN][K + 8]
-  const int ldb = K + 8;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int n0 = blockIdx.y * kBN;
-  // stage Bt rows n0 .. n0+63 (16-byte chunks)
-  const int chunks = kBN * K / 8;
-  for (int i = threadIdx.x; i < chunks; i += 256) {
-    const int r = i / (K / 8), c8 = i % (K / 8);
-    *reinterpret_cast<bf16x8 *>(&sB[r * ldb + c8 * 8]) = load8(Bt + (size_t)(n0 + r) * K + c8 * 8);
+template <int W, bool TRAIN>
+__global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Points pt, float *__restrict__ out,
+                                               float *__restrict__ lossp) {
+  constexpr int KS = W / 32, ld = W + kPad, kThreads = 2 * W;
+  constexpr int KM = KS > 4 ? KS : 4;  // the first layer has up to 128 inputs
+  extern __shared__ __align__(16) bf16 sm[];
+  const int nl = m.nl, K0 = m.K0, nin = m.nin, nout = m.nout, ld0 = K0 + kPad;
+  bf16 *sx = sm;                                 // [kTile][ld0]
+  bf16 *sd = sx + kTile * ld0;                   // training: output gradients, 2 x [kTile][ld]
+  bf16 *sh = sd + (TRAIN ? 2 * kTile * ld : 0);  // slots x [kTile][ld]
+  float *sy = reinterpret_cast<float *>(sh + (size_t)slots * kTile * ld);  // training: targets, [kTile][nout]
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int lp = lane / 16 * 4, ln = lane % 16;  // a lane's first point and column of a 16 x 16 result
+  const int p0 = blockIdx.x * kTile;
+  auto rows = [&](int j) { return sh + (size_t)(j % slots) * kTile * ld; };  // output of layer j
+
+  bf16x8 b[2 * KM];
+  load_frags<4>(b, m.wf, K0 / 32, W / 16, 2 * wave);
+
+  // inputs
+  if (pt.xs) {
+    for (int i = tid; i < kTile * K0 / 8; i += kThreads) {
+      const int p = i / (K0 / 8), c = i % (K0 / 8) * 8;
+      bf16x8 v = {};
+      if (p0 + p < pt.nv) v = load8(pt.xs + (size_t)pt.idx[p0 + p] * K0 + c);
+      *reinterpret_cast<bf16x8 *>(sx + p * ld0 + c) = v;
+    }
+  } else {
+    for (int i = tid; i < kTile * K0; i += kThreads) {
+      const int p = i / K0, c = i % K0;
+      sx[p * ld0 + c] = p0 + p < pt.nv && c < nin ? to_bf16(pt.x[(size_t)(p0 + p) * nin + c]) : (bf16)0;
+    }
   }
+  if (TRAIN)
+    for (int i = tid; i < kTile * nout; i += kThreads) {
+      const int p = p0 + i / nout;
+      float v = 0.0f;
+      if (p < pt.nv) v = pt.xs ? pt.ys[(size_t)pt.idx[p] * nout + i % nout] : pt.y[(size_t)p0 * nout + i];
+      sy[i] = v;
+    }
   __syncthreads();
-  const int p0 = blockIdx.x * kBP + wave * 32;
-  floatx4 acc[2][4];
-  for (int a = 0; a < 2; a++)
-    for (int t = 0; t < 4; t++) acc[a][t] = floatx4{0, 0, 0, 0};
-  const bf16 *a0p = A + (size_t)(p0 + lane % 16) * K + (lane / 16) * 8;
-  const bf16 *a1p = a0p + (size_t)16 * K;
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    const bf16x8 a0 = load8(a0p + k0), a1 = load8(a1p + k0);
-    for (int t = 0; t < 4; t++) {
-      const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(&sB[(t * 16 + lane % 16) * ldb + k0 + (lane / 16) * 8]);
-      acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bv, acc[0][t], 0, 0, 0);
-      acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, bv, acc[1][t], 0, 0, 0);
+  if (TRAIN) {
+    bf16 *xb = m.in;
+    for (int i = tid; i < kTile / 8 * K0; i += kThreads) {
+      const int q = i / K0, c = i % K0;
+      bf16x8 v;
+      for (int e = 0; e < 8; e++) v[e] = __builtin_bit_cast(__bf16, sx[(q * 8 + e) * ld0 + c]);
+      *reinterpret_cast<bf16x8 *>(xb + pt_index(p0 + q * 8, c, K0)) = v;
     }
   }
-  for (int a = 0; a < 2; a++)
-    for (int t = 0; t < 4; t++) {
-      const int n = n0 + t * 16 + lane % 16;
-      for (int r = 0; r < 4; r++) {
-        const int p = p0 + a * 16 + (lane / 16) * 4 + r;
-        const size_t o = (size_t)p * N + n;
-        if (EPI == 0) {
-          const float z = acc[a][t][r] + bias[n];
-          if (TRAIN) Z[o] = z;
-          const bf16 h = to_bf16(z * sigmoid(z));
-          H[o] = h;
-          if (TRAIN) Hb[((size_t)(p / 8) * N + n) * 8 + p % 8] = h;
-        } else {
-          const float z = Zp[o];
-          const float s = sigmoid(z);
-          const bf16 d = to_bf16(acc[a][t][r] * (s * (1.0f + z * (1.0f - s))));
-          H[o] = d;
-          Hb[((size_t)(p / 8) * N + n) * 8 + p % 8] = d;
+
+  // forward: hidden layers
+  floatx4 acc[2][2];
+  for (int l = 0; l < nl - 1; l++) {
+    float bl[2];
+    for (int t = 0; t < 2; t++) bl[t] = m.b[l * W + wave * 32 + t * 16 + ln];
+    if (l == 0)
+      product<4>(acc, sx, ld0, b, K0 / 32);
+    else
+      product<KS>(acc, rows(l - 1), ld, b, KS);
+    const bool last = l == nl - 2;  // (of the last layer every wave loads the two n tiles there are)
+    load_frags<KS>(b, m.wf + m.frag(l + 1), KS, last ? kOut / 16 : W / 16, last ? 0 : 2 * wave);
+    bf16 *h = rows(l), *hb = TRAIN ? m.in + m.inp(l + 1) : nullptr;
+    for (int i = 0; i < 2; i++)
+      for (int t = 0; t < 2; t++) {
+        float z[4], s[4];
+        for (int r = 0; r < 4; r++) z[r] = acc[i][t][r] + bl[t];
+        sigmoid4(z, s);
+        for (int r = 0; r < 4; r++) z[r] = z[r] * s[r];
+        put4(h, ld, hb, p0, W, i * 16 + lp, wave * 32 + t * 16 + ln, to_bf16x4(z));
+      }
+    __syncthreads();
+    if (TRAIN && l + slots <= nl - 2)
+      for (int i = tid; i < kTile * W / 8; i += kThreads) {
+        const int p = i / (W / 8), c = i % (W / 8) * 8;
+        *reinterpret_cast<bf16x8 *>(m.h + m.out(l) + (size_t)(p0 + p) * W + c) = load8(h + p * ld + c);
+      }
+  }
+
+  // last layer: wave 0 the first 16 points, wave 1 the others
+  float *sq = reinterpret_cast<float *>(sd + kTile * ld);  // squared errors, [kTile * kOut]
+  if (wave < 2) {
+    floatx4 o[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    const bf16 *r = rows(nl - 2) + (wave * 16 + ln) * ld + (lane / 16) * 8;
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+      const bf16x8 a = load8(r + s * 32);
+      for (int t = 0; t < 2; t++) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[2 * s + t], o[t], 0, 0, 0);
+    }
+    for (int t = 0; t < 2; t++) {
+      const int n = t * 16 + ln;
+      const float bn = n < nout ? m.b[(nl - 1) * W + n] : 0.0f;
+      float v[4];
+      for (int q = 0; q < 4; q++) {
+        const int p = wave * 16 + lp + q;
+        const bool real = p0 + p < pt.nv && n < nout;
+        const float z = o[t][q] + bn;
+        if (!TRAIN) {
+          if (real) out[(size_t)(p0 + p) * nout + n] = z;
+          continue;
         }
+        // loss = mean of squares; dZ = bf16(2 (z - y) / (nv nout)), zero on padding
+        float e2 = 0, g = 0;
+        if (real) {
+          const float e = z - sy[p * nout + n];
+          e2 = e * e;
+          g = 2.0f * e / ((float)pt.nv * (float)nout);
+        }
+        v[q] = g;
+        sq[p * kOut + n] = e2;
       }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Weight gradient partial of one chunk of kChunk points:
-// part[chunk][k][n] = sum_{p in chunk} X[p][k] dZ[p][n], 64 k x NT*16 n per
-// block (4 waves x 16 k), operands from the point-blocked copies.
-// ---------------------------------------------------------------------------
-template <int NT>
-__global__ __launch_bounds__(256) void k_bwd_weight(const bf16 *__restrict__ Xb, int K, const bf16 *__restrict__ dZb,
-                                                    int N, int P, float *__restrict__ part) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int k0 = blockIdx.x * 64 + wave * 16;
-  const int n0 = blockIdx.y * NT * 16;
-  const int pa = blockIdx.z * kChunk, pb = min(P, pa + kChunk);
-  floatx4 acc[NT];
-  for (int t = 0; t < NT; t++) acc[t] = floatx4{0, 0, 0, 0};
-  for (int p = pa; p < pb; p += 32) {
-    const size_t blk = (size_t)(p / 8) + lane / 16;
-    const bf16x8 a = load8(Xb + (blk * K + k0 + lane % 16) * 8);
-    for (int t = 0; t < NT; t++) {
-      const bf16x8 bv = load8(dZb + (blk * N + n0 + t * 16 + lane % 16) * 8);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[t], 0, 0, 0);
+      if (TRAIN) put4(sd, ld, m.dz + m.out(nl - 1), p0, kOut, wave * 16 + lp, n, to_bf16x4(v));
     }
   }
-  float *o = part + (size_t)blockIdx.z * K * N;
-  for (int t = 0; t < NT; t++)
-    for (int r = 0; r < 4; r++) {
-      const int k = k0 + (lane / 16) * 4 + r, n = n0 + t * 16 + lane % 16;
-      o[(size_t)k * N + n] = acc[t][r];
-    }
-}
-
-// bias-gradient partial of one chunk of kChunk points from the point-blocked
-// copy: block (chunk, 32 columns); thread (column c, j) sums the 8-point
-// blocks j, j + 8, ... of the chunk (16-byte loads), then the 8 partial sums
-// of a column are added in j order (reproducible).
-__global__ __launch_bounds__(256) void k_colsum(const bf16 *__restrict__ dZb, int N, int P, float *__restrict__ partb) {
-  __shared__ float sh[8][32];
-  const int c = threadIdx.x % 32, j = threadIdx.x / 32;
-  const int n = blockIdx.y * 32 + c;
-  const int pa = blockIdx.x * kChunk, pb = min(P, pa + kChunk);
-  float s = 0;
-  for (int b = pa / 8 + j; b < pb / 8; b += 8) {
-    const bf16x8 v = load8(dZb + ((size_t)b * N + n) * 8);
-    for (int e = 0; e < 8; e++) s += (float)v[e];
-  }
-  sh[j][c] = s;
+  if (!TRAIN) return;
+  bf16x8 c[2 * KS];
+  load_frags<1>(c, m.wb + m.frag(nl - 1), 1, W / 16, 2 * wave);
+  load_frags<KM>(b, m.wf + m.frag(nl - 2), m.K(nl - 2) / 32, W / 16, 2 * wave);
   __syncthreads();
-  if (j == 0) {
-    float t = 0;
-    for (int q = 0; q < 8; q++) t += sh[q][c];
-    partb[(size_t)blockIdx.x * N + n] = t;
-  }
-}
-
-// sum of nchunk partials in chunk order (loads batched ahead of the adds)
-__device__ __forceinline__ float chunk_sum(const float *__restrict__ part, int nchunk, long len, long i) {
-  float s = 0;
-  int c = 0;
-  for (; c + 8 <= nchunk; c += 8) {
-    float v[8];
-    for (int u = 0; u < 8; u++) v[u] = part[(size_t)(c + u) * len + i];
-    for (int u = 0; u < 8; u++) s += v[u];
-  }
-  for (; c < nchunk; c++) s += part[(size_t)c * len + i];
-  return s;
-}
-__global__ void k_sum_chunks(const float *__restrict__ part, int nchunk, long len, float *__restrict__ out) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= len) return;
-  out[i] = chunk_sum(part, nchunk, len, i);
-}
-
-// Loss and output gradient: out[P][No] (fp32), targets y[n][nout] of the
-// first nv points; dZ = bf16(2 (out - y) / (nv nout)) (zero on padding),
-// row-major and point-blocked; lossp[block] = partial sum of squares.
-__global__ __launch_bounds__(256) void k_loss(const float *__restrict__ out, int No, const float *__restrict__ y,
-                                              int nout, int nv, bf16 *__restrict__ dZ, bf16 *__restrict__ dZb,
-                                              float *__restrict__ lossp) {
-  __shared__ float sh[256];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;  // over P * No
-  const int p = i / No, n = i % No;
-  float sq = 0, g = 0;
-  if (p < nv && n < nout) {
-    const float e = out[i] - y[(size_t)p * nout + n];
-    sq = e * e;
-    g = 2.0f * e / ((float)nv * (float)nout);
-  }
-  const bf16 d = to_bf16(g);
-  dZ[i] = d;
-  dZb[((size_t)(p / 8) * No + n) * 8 + p % 8] = d;
-  sh[threadIdx.x] = sq;
-  __syncthreads();
+  // the sums of squares of 8 points each, by a fixed tree
   for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+    for (int i = tid; i < kTile / 8 * w; i += kThreads) {
+      float *s = sq + i / w * 256 + i % w;
+      s[0] += s[w];
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) lossp[blockIdx.x] = sh[0];
+  if (tid < kTile / 8) lossp[blockIdx.x * (kTile / 8) + tid] = sq[tid * 256];
+  __syncthreads();  // the second gradient buffer holds the squares no longer
+
+  // backward: dZ of layer l - 1 from dZ of layer l
+  for (int l = nl - 1; l >= 1; l--) {
+    const bf16 *cur = sd + ((nl - 1 - l) & 1) * kTile * ld;
+    bf16 *nxt = sd + ((nl - l) & 1) * kTile * ld;
+    if (l >= 2 && l - 2 + slots <= nl - 2) {  // the input rows of layer l - 1 have left LDS
+      bf16 *h = rows(l - 2);
+      for (int i = tid; i < kTile * W / 8; i += kThreads) {
+        const int p = i / (W / 8), k = i % (W / 8) * 8;
+        *reinterpret_cast<bf16x8 *>(h + p * ld + k) = load8(m.h + m.out(l - 2) + (size_t)(p0 + p) * W + k);
+      }
+      __syncthreads();
+    }
+    float bl[2];
+    for (int t = 0; t < 2; t++) bl[t] = m.b[(l - 1) * W + wave * 32 + t * 16 + ln];
+    floatx4 z4[2][2];
+    if (l == nl - 1)
+      product<1>(acc, cur, ld, c, 1);
+    else
+      product<KS>(acc, cur, ld, c, KS);
+    if (l == 1)
+      product<4>(z4, sx, ld0, b, K0 / 32);
+    else
+      product<KS>(z4, rows(l - 2), ld, b, KS);
+    const int j = max(l - 2, 0);  // (the last round loads what it does not use)
+    load_frags<KS>(c, m.wb + m.frag(j + 1), m.N(j + 1) / 32, W / 16, 2 * wave);
+    load_frags<KM>(b, m.wf + m.frag(j), m.K(j) / 32, W / 16, 2 * wave);
+    for (int i = 0; i < 2; i++)
+      for (int t = 0; t < 2; t++) {
+        float z[4], s[4];
+        for (int r = 0; r < 4; r++) z[r] = z4[i][t][r] + bl[t];
+        sigmoid4(z, s);
+        for (int r = 0; r < 4; r++) z[r] = acc[i][t][r] * (s[r] * (1.0f + z[r] * (1.0f - s[r])));
+        put4(nxt, ld, m.dz + m.out(l - 1), p0, W, i * 16 + lp, wave * 32 + t * 16 + ln, to_bf16x4(z));
+      }
+    __syncthreads();
+  }
 }
 
-// out[slot] = scale * (sum of n partials): one block, thread t sums
-// t, t + 256, ... then a fixed tree (reproducible)
-__global__ __launch_bounds__(256) void k_sum_small(const float *__restrict__ part, int n, float scale,
-                                                   float *__restrict__ out, int slot) {
+// ---------------------------------------------------------------------------
+// k_weights: weight and bias gradients of every layer from the inputs and
+// output gradients, and Adam on them (or the gradients themselves).
+// A block owns 32 k x 64 n (32 k x 32 n of the last layer) over all points,
+// a wave 32 k x 32 n: partial products of kChunk points (32 at a time, in
+// MFMA order), added in chunk order, so the result does not depend on the
+// launch.  Operands go straight from memory to registers, kFlight steps of 32
+// points ahead.  The bias sums are blocks of their own (beside a block's
+// products they took as long again).  Blocks of one layer share an XCD (block b: XCD b % 8, layer b % 8 of each eight), so its
+// L2 reads each operand once.  Adam runs on the sum while it is in registers:
+// FP32 master weights, then the BF16 fragments of the next step's products.
+// Bound by the operands' way from L2 into the CUs, 8 KB per block and 32
+// points (with every block on the same 16 steps it takes 5 us less; 8 to 24
+// steps in flight make no difference).  Measured at 8 x 256, 16384 points: 60
+// us, against 192 us for a launch per layer for the partial products, the bias
+// sums and each update, with the partial products in memory.
+// ---------------------------------------------------------------------------
+struct WeightTile {
+  int layer, k0, n0;  // layer -1: no work; k0 -1: the bias sums of 16 columns
+};
+struct AdamStep {
+  float lr, c1, c2;
+};
+struct Moments {
+  float *m1, *m2, *m1b, *m2b;
+};
+constexpr int kFlight = 16;
+
+// One Adam step on parameter p[o].
+__device__ __forceinline__ float adam(float *p, float *m1, float *m2, size_t o, float g, const AdamStep &st) {
+  const float a = 0.9f * m1[o] + 0.1f * g;
+  const float v = 0.999f * m2[o] + 0.001f * g * g;
+  m1[o] = a;
+  m2[o] = v;
+  const float x = p[o] - st.lr * (a / st.c1) / (sqrtf(v / st.c2) + 1e-8f);
+  p[o] = x;
+  return x;
+}
+
+// Bias gradients of columns n0 .. n0 + 15 of layer l (two waves): a lane takes
+// one column of one chunk, sums the 8-point blocks j, j + 8, ... of the chunk
+// for each j, then the eight sums, and the chunks add up in order.
+template <bool ADAM>
+__device__ __forceinline__ void bias_sums(const Net &m, int l, int n0, const AdamStep &st, const Moments &mo,
+                                          float *gb) {
+  __shared__ float part[8][16];
+  const int tid = threadIdx.x, N = m.N(l), c0 = tid / 16, nblk = (int)(m.P / 8);
+  const bf16 *d = m.dz + m.out(l);
+  float sum = 0.0f;
+  for (int b0 = 0; b0 < nblk; b0 += 8 * (kChunk / 8)) {
+    const int b = b0 + c0 * (kChunk / 8);
+    float s[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) s[j] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kChunk / 64; i++)
+      if (b + 8 * i < nblk) {
+        bf16x8 v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = load8(d + pt_index((long)(b + 8 * i + j) * 8, n0 + tid % 16, N));
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          for (int e = 0; e < 8; e++) s[j] += (float)v[j][e];
+      }
+    float t = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) t += s[j];
+    part[c0][tid % 16] = t;
+    __syncthreads();
+    if (tid < 16)
+      for (int c = 0; c < 8; c++)
+        if (b0 + c * (kChunk / 8) < nblk) sum += part[c][tid];
+    __syncthreads();
+  }
+  if (tid >= 16 || n0 + tid >= m.n(l)) return;
+  const size_t o = m.ob(l) + n0 + tid;
+  if (ADAM)
+    adam(m.b, mo.m1b, mo.m2b, o, sum, st);
+  else
+    gb[o] = sum;
+}
+
+template <bool ADAM>
+__global__ __launch_bounds__(128, 1) void k_weights(const Net m, const WeightTile *__restrict__ tiles,
+                                                    const AdamStep st, const Moments mo, float *__restrict__ gw,
+                                                    float *__restrict__ gb) {
+  const WeightTile tl = tiles[blockIdx.x];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int l = tl.layer, n0 = tl.n0 + wave * 32;
+  if (l < 0) return;
+  if (tl.k0 < 0) {
+    bias_sums<ADAM>(m, l, tl.n0, st, mo, gb);
+    return;
+  }
+  const int K = m.K(l), N = m.N(l), rk = m.k(l), rn = m.n(l);
+  if (n0 >= N) return;
+  const int nstep = (int)(m.P / 32);  // a multiple of 4
+  // the step to load next (its last one again past the end): uniform bases
+  // and a lane's offset, so that a step costs a few scalar additions
+  const bf16 *x = m.in + m.inp(l) + tl.k0 / 16 * 512, *d = m.dz + m.out(l) + n0 / 16 * 512;
+  int left = nstep - 1;
+  bf16x8 a[kFlight][2], b[kFlight][2];
+  auto fetch = [&](int slot) {
+    for (int t = 0; t < 2; t++) {
+      a[slot][t] = load8(x + lane * 8 + t * 512);
+      b[slot][t] = load8(d + lane * 8 + t * 512);
+    }
+    x += left > 0 ? 32 * K : 0;
+    d += left > 0 ? 32 * N : 0;
+    left--;
+  };
+  floatx4 acc[2][2], sum[2][2];
+  for (int i = 0; i < 2; i++)
+    for (int t = 0; t < 2; t++) acc[i][t] = sum[i][t] = floatx4{0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < kFlight; i++) fetch(i);
+  for (int s0 = 0; s0 < nstep; s0 += kFlight) {
+#pragma unroll
+    for (int g = 0; g < kFlight / 4; g++) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int i = g * 4 + q;
+        if (s0 + g * 4 < nstep)
+          for (int u = 0; u < 2; u++)
+            for (int t = 0; t < 2; t++)
+              acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][u], b[i][t], acc[u][t], 0, 0, 0);
+        fetch(i);
+      }
+      const int done = s0 + g * 4 + 4;  // steps done
+      if (done <= nstep && (done % (kChunk / 32) == 0 || done == nstep)) {
+        for (int u = 0; u < 2; u++)
+          for (int t = 0; t < 2; t++)
+            for (int r = 0; r < 4; r++) {
+              sum[u][t][r] += acc[u][t][r];
+              acc[u][t][r] = 0.0f;
+            }
+      }
+    }
+  }
+  for (int u = 0; u < 2; u++)
+    for (int t = 0; t < 2; t++)
+      for (int r = 0; r < 4; r++) {
+        const int k = tl.k0 + u * 16 + lane / 16 * 4 + r, n = n0 + t * 16 + lane % 16;
+        if (k >= rk || n >= rn) continue;
+        const size_t o = m.ow(l) + (size_t)k * rn + n;
+        const float gi = sum[u][t][r];
+        if (!ADAM) {
+          gw[o] = gi;
+          continue;
+        }
+        const bf16 h = to_bf16(adam(m.w, mo.m1, mo.m2, o, gi, st));
+        m.wf[m.frag(l) + wf_index(k, n, N)] = h;
+        m.wb[m.frag(l) + wb_index(k, n, K)] = h;
+      }
+}
+
+// Batch losses of an epoch, one block per step: scale * (sum of the step's n
+// partials), thread t summing t, t + 256, ... then a fixed tree (reproducible).
+__global__ __launch_bounds__(256) void k_losses(const float *__restrict__ part, int n, float scale, float scale_last,
+                                                float *__restrict__ out) {
   __shared__ double sh[256];
+  part += (size_t)blockIdx.x * n;
   double a = 0;
   for (int i = threadIdx.x; i < n; i += 256) a += part[i];
   sh[threadIdx.x] = a;
@@ -310,53 +553,7 @@ __global__ __launch_bounds__(256) void k_sum_small(const float *__restrict__ par
     if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[slot] = (float)(sh[0] * scale);
-}
-
-// Batch assembly: rows idx[start + i] of the resident set (bf16 inputs padded
-// to Kp, fp32 targets), zero rows past n; also the point-blocked input copy.
-__global__ __launch_bounds__(256) void k_gather(const bf16 *__restrict__ xs, int Kp, const float *__restrict__ ys,
-                                                int nout, const int *__restrict__ idx, int nv, int P,
-                                                bf16 *__restrict__ X, bf16 *__restrict__ Xb, float *__restrict__ Y) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;  // over P * Kp
-  if (i >= (long)P * Kp) return;
-  const int p = (int)(i / Kp), k = (int)(i % Kp);
-  bf16 v = 0;
-  if (p < nv) v = xs[(size_t)idx[p] * Kp + k];
-  X[i] = v;
-  Xb[((size_t)(p / 8) * Kp + k) * 8 + p % 8] = v;
-  if (k < nout) Y[(size_t)p * nout + k] = p < nv ? ys[(size_t)idx[p] * nout + k] : 0.0f;
-}
-
-// Adam on one layer (FP32 master weights, padded K x N) straight from the
-// chunk partials of its gradients (summed in chunk order, as k_sum_chunks
-// forms them), then the BF16 copies W[k][n] and Wt[n][k].
-__global__ void k_adam_w_part(float *w, const float *part, int nchunk, float *m1, float *m2, int K, int N, float lr,
-                              float c1, float c2, bf16 *W, bf16 *Wt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= K * N) return;
-  const float gi = chunk_sum(part, nchunk, (long)K * N, i);
-  const float a = 0.9f * m1[i] + 0.1f * gi;
-  const float v = 0.999f * m2[i] + 0.001f * gi * gi;
-  m1[i] = a;
-  m2[i] = v;
-  const float wi = w[i] - lr * (a / c1) / (sqrtf(v / c2) + 1e-8f);
-  w[i] = wi;
-  const int k = i / N, n = i % N;
-  const bf16 h = to_bf16(wi);
-  W[i] = h;
-  Wt[(size_t)n * K + k] = h;
-}
-__global__ void k_adam_b_part(float *b, const float *partb, int nchunk, float *m1, float *m2, int n, float lr,
-                              float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = chunk_sum(partb, nchunk, n, i);
-  const float a = 0.9f * m1[i] + 0.1f * gi;
-  const float v = 0.999f * m2[i] + 0.001f * gi * gi;
-  m1[i] = a;
-  m2[i] = v;
-  b[i] = b[i] - lr * (a / c1) / (sqrtf(v / c2) + 1e-8f);
+  if (threadIdx.x == 0) out[blockIdx.x] = (float)(sh[0] * (blockIdx.x == gridDim.x - 1 ? scale_last : scale));
 }
 
 __global__ void k_mfma_check(const bf16 *a, const bf16 *b, float *d) {
@@ -373,15 +570,24 @@ __global__ void k_mfma_check(const bf16 *a, const bf16 *b, float *d) {
   for (int r = 0; r < 4; r++) d[((lane / 16) * 4 + r) * 16 + lane % 16] = c[r];
 }
 
+// BF16 fragments of a layer's weights (blockIdx.y) from the FP32 masters; the
+// padding stays zero.
+__global__ __launch_bounds__(256) void k_pack(const Net m) {
+  const int l = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= m.k(l) * m.n(l)) return;
+  const int k = i / m.n(l), n = i % m.n(l);
+  const bf16 h = to_bf16(m.w[m.ow(l) + i]);
+  m.wf[m.frag(l) + wf_index(k, n, m.N(l))] = h;
+  m.wb[m.frag(l) + wb_index(k, n, m.K(l))] = h;
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-struct Layer {
-  int K = 0, N = 0;     // padded fan-in, fan-out
-  int k = 0, n = 0;     // real
-  float *w = nullptr, *b = nullptr, *gw = nullptr, *gb = nullptr;
-  float *m1w = nullptr, *m2w = nullptr, *m1b = nullptr, *m2b = nullptr;
-  bf16 *W = nullptr, *Wt = nullptr;
+// A device buffer that grows and is kept for the next call.
+struct Buf {
+  void *p = nullptr;
+  size_t bytes = 0;
 };
 
 }  // namespace usgmlp
@@ -390,25 +596,24 @@ using namespace usgmlp;
 
 struct usg_mlp {
   usg_mlp_desc d{};
-  std::vector<Layer> L;
+  long nw = 0, nb = 0;
+  Net net{};
+  Moments mo{};
   hipStream_t s = nullptr;
   std::vector<void *> allocs;
   long step = 0;
-  // batch buffers (capacity P points)
+  WeightTile *d_tiles = nullptr;
+  int ntiles = 0;
+  int slots = 0;              // layers whose rows LDS holds in training
+  size_t lds_train = 0, lds_predict = 0;
+  // training buffers for `cap` points (Net's in, dz and h)
   int cap = 0;
   std::vector<void *> bufs;
-  bf16 *X = nullptr, *Xb = nullptr;
-  std::vector<float *> Z;           // per layer [P][N]
-  std::vector<bf16 *> H, Hb;        // per hidden layer output [P][N] row / blocked
-  bf16 *dA = nullptr, *dAb = nullptr, *dB = nullptr, *dBb = nullptr;  // dZ ping-pong
-  float *Y = nullptr, *lossp = nullptr, *part = nullptr, *partb = nullptr;
+  Buf x, y, g, lossp, losses, idx;
   // resident training set
   bf16 *xs = nullptr;
   float *ys = nullptr;
-  int *idx = nullptr;
-  long nset = 0, idx_cap = 0;
-  float *lossbuf = nullptr;  // per-step batch losses of an epoch
-  long lossbuf_cap = 0;
+  long nset = 0;
 };
 
 namespace usgmlp {
@@ -422,119 +627,87 @@ int dalloc(std::vector<void *> &v, T **p, size_t n) {
   return 0;
 }
 
-int free_bufs(usg_mlp *m) {
-  for (void *p : m->bufs) hipFree(p);
-  m->bufs.clear();
-  m->cap = 0;
-  return 0;
-}
-
-int ensure_cap(usg_mlp *m, int P) {
-  if (P <= m->cap) return 0;
+int grow(usg_mlp *m, Buf &b, size_t bytes) {
+  if (bytes <= b.bytes) return 0;
   HIPCHK(hipStreamSynchronize(m->s));
-  free_bufs(m);
-  const int nl = (int)m->L.size();
-  const int K0 = m->L[0].K, W = m->d.width, No = m->L.back().N;
-  auto &v = m->bufs;
-  int rc = 0;
-  rc |= dalloc(v, &m->X, (size_t)P * K0);
-  rc |= dalloc(v, &m->Xb, (size_t)P * K0);
-  m->Z.assign(nl, nullptr);
-  m->H.assign(nl, nullptr);
-  m->Hb.assign(nl, nullptr);
-  for (int l = 0; l < nl; l++) {
-    rc |= dalloc(v, &m->Z[l], (size_t)P * m->L[l].N);
-    if (l < nl - 1) {
-      rc |= dalloc(v, &m->H[l], (size_t)P * W);
-      rc |= dalloc(v, &m->Hb[l], (size_t)P * W);
-    }
-  }
-  const int mx = std::max(W, No);
-  rc |= dalloc(v, &m->dA, (size_t)P * mx);
-  rc |= dalloc(v, &m->dAb, (size_t)P * mx);
-  rc |= dalloc(v, &m->dB, (size_t)P * mx);
-  rc |= dalloc(v, &m->dBb, (size_t)P * mx);
-  rc |= dalloc(v, &m->Y, (size_t)P * m->d.nout);
-  rc |= dalloc(v, &m->lossp, (size_t)P * No / 256 + 1);
-  const int nch = (P + kChunk - 1) / kChunk;
-  rc |= dalloc(v, &m->part, (size_t)nch * std::max(K0, W) * std::max(W, No));
-  rc |= dalloc(v, &m->partb, (size_t)nch * mx);
-  if (rc) return rc;
-  m->cap = P;
+  if (b.p) hipFree(b.p);
+  b.p = nullptr;
+  b.bytes = 0;
+  HIPCHK(hipMalloc(&b.p, bytes));
+  b.bytes = bytes;
   return 0;
 }
 
 int round_up(int a, int b) { return (a + b - 1) / b * b; }
 
-// forward over P (multiple of 64) points already in m->X
-void forward(usg_mlp *m, int P, bool train) {
-  const int nl = (int)m->L.size();
-  const bf16 *x = m->X;
-  for (int l = 0; l < nl; l++) {
-    const Layer &y = m->L[l];
-    const bool last = l == nl - 1;
-    if (last) {
-      const int NT = 2;
-      hipLaunchKernelGGL((k_fwd<NT, false, false>), dim3(P / 64, y.N / (NT * 16)), dim3(256), 0, m->s, x, y.K,
-                         y.Wt, y.b, y.N, m->Z[l], nullptr, nullptr);
-    } else if (train) {
-      hipLaunchKernelGGL((k_gemm<0, true>), dim3(P / kBP, y.N / kBN), dim3(256), kBN * (y.K + 8) * 2, m->s, x, y.K,
-                         y.Wt, y.b, y.N, nullptr, m->Z[l], m->H[l], m->Hb[l]);
-    } else {
-      hipLaunchKernelGGL((k_gemm<0, false>), dim3(P / kBP, y.N / kBN), dim3(256), kBN * (y.K + 8) * 2, m->s, x, y.K,
-                         y.Wt, y.b, y.N, nullptr, nullptr, m->H[l], nullptr);
-    }
-    x = m->H[l];
+// Training buffers for P points (a multiple of 128).
+int ensure_cap(usg_mlp *m, int P) {
+  Net &t = m->net;
+  t.P = P;
+  if (P <= m->cap) return 0;
+  HIPCHK(hipStreamSynchronize(m->s));
+  for (void *p : m->bufs) hipFree(p);
+  m->bufs.clear();
+  m->cap = 0;
+  int rc = 0;
+  if ((rc = dalloc(m->bufs, &t.in, (size_t)t.inp(t.nl))) ||
+      (rc = dalloc(m->bufs, &t.dz, (size_t)t.out(t.nl - 1) + (size_t)P * kOut)) ||
+      (m->slots < t.nl - 1 && (rc = dalloc(m->bufs, &t.h, (size_t)t.out(t.nl - 1)))))
+    return rc;
+  m->cap = P;
+  return 0;
+}
+
+template <int W>
+int net_lds(usg_mlp *m, int limit) {
+  const size_t row = (size_t)kTile * (W + kPad) * sizeof(bf16), x = (size_t)kTile * (m->net.K0 + kPad) * sizeof(bf16),
+               y = (size_t)kTile * m->d.nout * sizeof(float);
+  m->slots = std::min<int>(m->net.nl - 1, (int)(((size_t)limit - x - y) / row) - 2);
+  m->slots = std::max(m->slots, 2);
+  m->lds_train = x + y + (2 + m->slots) * row;
+  m->lds_predict = x + 2 * row;
+  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_net<W, true>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)m->lds_train));
+  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_net<W, false>),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)m->lds_predict));
+  return 0;
+}
+
+template <int W>
+void launch_net(usg_mlp *m, bool train, int blocks, const Points &pt, float *out, float *lossp) {
+  if (train)
+    hipLaunchKernelGGL((k_net<W, true>), dim3(blocks), dim3(2 * W), m->lds_train, m->s, m->net, m->slots, pt, out,
+                       lossp);
+  else
+    hipLaunchKernelGGL((k_net<W, false>), dim3(blocks), dim3(2 * W), m->lds_predict, m->s, m->net, 2, pt, out, lossp);
+}
+
+void net(usg_mlp *m, bool train, int blocks, const Points &pt, float *out, float *lossp) {
+  switch (m->d.width) {
+    case 64: launch_net<64>(m, train, blocks, pt, out, lossp); break;
+    case 128: launch_net<128>(m, train, blocks, pt, out, lossp); break;
+    case 192: launch_net<192>(m, train, blocks, pt, out, lossp); break;
+    default: launch_net<256>(m, train, blocks, pt, out, lossp); break;
   }
 }
 
-// Adam step parameters (training); null in the gradient-only path
-struct AdamStep {
-  float lr, c1, c2;
-};
-
-// backward from the output gradient in dA/dAb: gradients into L[l].gw/gb,
-// or, with an Adam step, each layer updated right after its last use (the
-// data-gradient product reads W_l before W_l changes)
-void backward(usg_mlp *m, int P, const AdamStep *adam = nullptr) {
-  const int nl = (int)m->L.size();
-  const int nch = (P + kChunk - 1) / kChunk;
-  bf16 *cur = m->dA, *curb = m->dAb, *nxt = m->dB, *nxtb = m->dBb;
-  for (int l = nl - 1; l >= 0; l--) {
-    Layer &y = m->L[l];
-    const bf16 *inb = l == 0 ? m->Xb : m->Hb[l - 1];
-    // N is 32 (output layer: 2 column tiles of 16) or a multiple of 64 (4 tiles)
-    if (y.N % 64 == 0)
-      hipLaunchKernelGGL((k_bwd_weight<4>), dim3(y.K / 64, y.N / 64, nch), dim3(256), 0, m->s, inb, y.K, curb, y.N,
-                         P, m->part);
-    else
-      hipLaunchKernelGGL((k_bwd_weight<2>), dim3(y.K / 64, y.N / 32, nch), dim3(256), 0, m->s, inb, y.K, curb, y.N,
-                         P, m->part);
-    hipLaunchKernelGGL(k_colsum, dim3(nch, y.N / 32), dim3(256), 0, m->s, curb, y.N, P, m->partb);
-    if (!adam) {
-      hipLaunchKernelGGL(k_sum_chunks, dim3((y.K * y.N + 255) / 256), dim3(256), 0, m->s, m->part, nch,
-                         (long)y.K * y.N, y.gw);
-      hipLaunchKernelGGL(k_sum_chunks, dim3(1), dim3(256), 0, m->s, m->partb, nch, (long)y.N, y.gb);
-    }
-    if (l > 0) {
-      if (y.N % 32 == 0 && y.N >= 64)
-        // dH = dZ W^T: A = dZ [P][N], Bt = W [K][N] (rows = outputs k)
-        hipLaunchKernelGGL((k_gemm<1, true>), dim3(P / kBP, y.K / kBN), dim3(256), kBN * (y.N + 8) * 2, m->s, cur,
-                           y.N, y.W, nullptr, y.K, m->Z[l - 1], nullptr, nxt, nxtb);
-      else
-        hipLaunchKernelGGL((k_bwd_data<2>), dim3(P / 64, y.K / 32), dim3(256), 0, m->s, cur, y.N, y.W, y.K,
-                           m->Z[l - 1], nxt, nxtb);
-    }
-    if (adam) {
-      hipLaunchKernelGGL(k_adam_w_part, dim3((y.K * y.N + 255) / 256), dim3(256), 0, m->s, y.w, m->part, nch, y.m1w,
-                         y.m2w, y.K, y.N, adam->lr, adam->c1, adam->c2, y.W, y.Wt);
-      hipLaunchKernelGGL(k_adam_b_part, dim3((y.N + 255) / 256), dim3(256), 0, m->s, y.b, m->partb, nch, y.m1b, y.m2b,
-                         y.N, adam->lr, adam->c1, adam->c2);
-    }
-    if (l == 0) break;
-    std::swap(cur, nxt);
-    std::swap(curb, nxtb);
-  }
+// The blocks of k_weights: block b works on a layer l with l % 8 == b % 8, so
+// that a layer's blocks run on one XCD.
+int build_tiles(usg_mlp *m) {
+  std::vector<WeightTile> by[8], all;
+  for (int l = 0; l < m->net.nl; l++)
+    for (int k0 = 0; k0 < m->net.K(l); k0 += 32)
+      for (int n0 = 0; n0 < m->net.N(l); n0 += 64) by[l % 8].push_back({l, k0, n0});
+  for (int l = 0; l < m->net.nl; l++)
+    for (int n0 = 0; n0 < m->net.n(l); n0 += 16) by[l % 8].push_back({l, -1, n0});
+  size_t most = 0;
+  for (auto &v : by) most = std::max(most, v.size());
+  for (size_t i = 0; i < most; i++)
+    for (auto &v : by) all.push_back(i < v.size() ? v[i] : WeightTile{-1, 0, 0});
+  m->ntiles = (int)all.size();
+  if (int rc = dalloc(m->allocs, &m->d_tiles, all.size())) return rc;
+  HIPCHK(hipMemcpy(m->d_tiles, all.data(), all.size() * sizeof(WeightTile), hipMemcpyHostToDevice));
+  return 0;
 }
 
 }  // namespace usgmlp
@@ -556,15 +729,43 @@ int usg_mlp_sizes(const usg_mlp_desc *d, long *nw, long *nb) {
 int usg_mlp_destroy(usg_mlp *m) {
   if (!m) return 0;
   if (m->s) hipStreamSynchronize(m->s);
-  free_bufs(m);
+  for (void *p : m->bufs) hipFree(p);
   for (void *p : m->allocs) hipFree(p);
+  for (Buf *b : {&m->x, &m->y, &m->g, &m->lossp, &m->losses, &m->idx})
+    if (b->p) hipFree(b->p);
   if (m->xs) hipFree(m->xs);
   if (m->ys) hipFree(m->ys);
-  if (m->idx) hipFree(m->idx);
-  if (m->lossbuf) hipFree(m->lossbuf);
   if (m->s) hipStreamDestroy(m->s);
   delete m;
   return 0;
+}
+
+static int create(usg_mlp *m) {
+  const usg_mlp_desc &d = m->d;
+  HIPCHK(hipStreamCreate(&m->s));
+  Net &t = m->net;
+  t.nl = d.nlayer;
+  t.W = d.width;
+  t.K0 = round_up(d.nin, 64);
+  t.nin = d.nin;
+  t.nout = d.nout;
+  const size_t frags = t.frag(t.nl - 1) + (size_t)t.W * kOut;
+  int rc = 0, dev = 0, limit = 0;
+  if ((rc = dalloc(m->allocs, &t.wf, frags)) || (rc = dalloc(m->allocs, &t.wb, frags)) ||
+      (rc = dalloc(m->allocs, &t.w, m->nw)) || (rc = dalloc(m->allocs, &t.b, m->nb)) ||
+      (rc = dalloc(m->allocs, &m->mo.m1, m->nw)) || (rc = dalloc(m->allocs, &m->mo.m2, m->nw)) ||
+      (rc = dalloc(m->allocs, &m->mo.m1b, m->nb)) || (rc = dalloc(m->allocs, &m->mo.m2b, m->nb)) ||
+      (rc = build_tiles(m)))
+    return rc;
+  for (bf16 *p : {t.wf, t.wb}) HIPCHK(hipMemsetAsync(p, 0, frags * sizeof(bf16), m->s));
+  HIPCHK(hipGetDevice(&dev));
+  HIPCHK(hipDeviceGetAttribute(&limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  switch (d.width) {
+    case 64: return net_lds<64>(m, limit);
+    case 128: return net_lds<128>(m, limit);
+    case 192: return net_lds<192>(m, limit);
+    default: return net_lds<256>(m, limit);
+  }
 }
 
 int usg_mlp_create(const usg_mlp_desc *d, usg_mlp **out) {
@@ -577,67 +778,27 @@ int usg_mlp_create(const usg_mlp_desc *d, usg_mlp **out) {
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return fail(-2, "no GPU visible");
   usg_mlp *m = new usg_mlp();
   m->d = *d;
-  if (hipStreamCreate(&m->s) != hipSuccess) {
-    delete m;
-    return fail(-3, "hipStreamCreate");
-  }
-  m->L.resize(d->nlayer);
-  for (int l = 0; l < d->nlayer; l++) {
-    Layer &y = m->L[l];
-    y.k = l == 0 ? d->nin : d->width;
-    y.n = l == d->nlayer - 1 ? d->nout : d->width;
-    y.K = l == 0 ? round_up(d->nin, 64) : d->width;
-    y.N = l == d->nlayer - 1 ? 32 : d->width;
-    const size_t kn = (size_t)y.K * y.N;
-    rc = 0;
-    rc |= dalloc(m->allocs, &y.w, kn);
-    rc |= dalloc(m->allocs, &y.gw, kn);
-    rc |= dalloc(m->allocs, &y.m1w, kn);
-    rc |= dalloc(m->allocs, &y.m2w, kn);
-    rc |= dalloc(m->allocs, &y.b, y.N);
-    rc |= dalloc(m->allocs, &y.gb, y.N);
-    rc |= dalloc(m->allocs, &y.m1b, y.N);
-    rc |= dalloc(m->allocs, &y.m2b, y.N);
-    rc |= dalloc(m->allocs, &y.W, kn);
-    rc |= dalloc(m->allocs, &y.Wt, kn);
-    if (rc) {
-      usg_mlp_destroy(m);
-      return rc;
-    }
-  }
-  *out = m;
+  m->nw = nw;
+  m->nb = nb;
   // zero parameters until set
   std::vector<float> w(nw, 0.0f), b(nb, 0.0f);
-  return usg_mlp_set_params(m, w.data(), b.data());
+  if ((rc = create(m)) || (rc = usg_mlp_set_params(m, w.data(), b.data()))) {
+    usg_mlp_destroy(m);
+    return rc;
+  }
+  *out = m;
+  return 0;
 }
 
 int usg_mlp_set_params(usg_mlp *m, const float *w, const float *b) {
   if (!m || !w || !b) return fail(-1, "null argument");
-  long ow = 0, ob = 0;
-  for (Layer &y : m->L) {
-    std::vector<float> pw((size_t)y.K * y.N, 0.0f), pb(y.N, 0.0f);
-    std::vector<bf16> W((size_t)y.K * y.N), Wt((size_t)y.K * y.N);
-    for (int k = 0; k < y.k; k++)
-      for (int n = 0; n < y.n; n++) pw[(size_t)k * y.N + n] = w[ow + (long)k * y.n + n];
-    for (int n = 0; n < y.n; n++) pb[n] = b[ob + n];
-    ow += (long)y.k * y.n;
-    ob += y.n;
-    for (int k = 0; k < y.K; k++)
-      for (int n = 0; n < y.N; n++) {
-        const bf16 h = to_bf16(pw[(size_t)k * y.N + n]);
-        W[(size_t)k * y.N + n] = h;
-        Wt[(size_t)n * y.K + k] = h;
-      }
-    const size_t kn = (size_t)y.K * y.N;
-    HIPCHK(hipMemcpyAsync(y.w, pw.data(), kn * 4, hipMemcpyHostToDevice, m->s));
-    HIPCHK(hipMemcpyAsync(y.b, pb.data(), y.N * 4, hipMemcpyHostToDevice, m->s));
-    HIPCHK(hipMemcpyAsync(y.W, W.data(), kn * 2, hipMemcpyHostToDevice, m->s));
-    HIPCHK(hipMemcpyAsync(y.Wt, Wt.data(), kn * 2, hipMemcpyHostToDevice, m->s));
-    HIPCHK(hipMemsetAsync(y.m1w, 0, kn * 4, m->s));
-    HIPCHK(hipMemsetAsync(y.m2w, 0, kn * 4, m->s));
-    HIPCHK(hipMemsetAsync(y.m1b, 0, y.N * 4, m->s));
-    HIPCHK(hipMemsetAsync(y.m2b, 0, y.N * 4, m->s));
-  }
+  HIPCHK(hipMemcpyAsync(m->net.w, w, m->nw * sizeof(float), hipMemcpyHostToDevice, m->s));
+  HIPCHK(hipMemcpyAsync(m->net.b, b, m->nb * sizeof(float), hipMemcpyHostToDevice, m->s));
+  for (float *p : {m->mo.m1, m->mo.m2}) HIPCHK(hipMemsetAsync(p, 0, m->nw * sizeof(float), m->s));
+  for (float *p : {m->mo.m1b, m->mo.m2b}) HIPCHK(hipMemsetAsync(p, 0, m->nb * sizeof(float), m->s));
+  const int most = std::max(m->d.nin, m->d.width) * m->d.width;
+  hipLaunchKernelGGL(k_pack, dim3((most + 255) / 256, m->net.nl), dim3(256), 0, m->s, m->net);
+  HIPCHK(hipGetLastError());
   m->step = 0;
   HIPCHK(hipStreamSynchronize(m->s));
   return 0;
@@ -645,111 +806,61 @@ int usg_mlp_set_params(usg_mlp *m, const float *w, const float *b) {
 
 int usg_mlp_get_params(usg_mlp *m, float *w, float *b) {
   if (!m || !w || !b) return fail(-1, "null argument");
-  long ow = 0, ob = 0;
-  for (Layer &y : m->L) {
-    std::vector<float> pw((size_t)y.K * y.N), pb(y.N);
-    HIPCHK(hipMemcpyAsync(pw.data(), y.w, pw.size() * 4, hipMemcpyDeviceToHost, m->s));
-    HIPCHK(hipMemcpyAsync(pb.data(), y.b, pb.size() * 4, hipMemcpyDeviceToHost, m->s));
-    HIPCHK(hipStreamSynchronize(m->s));
-    for (int k = 0; k < y.k; k++)
-      for (int n = 0; n < y.n; n++) w[ow + (long)k * y.n + n] = pw[(size_t)k * y.N + n];
-    for (int n = 0; n < y.n; n++) b[ob + n] = pb[n];
-    ow += (long)y.k * y.n;
-    ob += y.n;
-  }
+  HIPCHK(hipMemcpyAsync(w, m->net.w, m->nw * sizeof(float), hipMemcpyDeviceToHost, m->s));
+  HIPCHK(hipMemcpyAsync(b, m->net.b, m->nb * sizeof(float), hipMemcpyDeviceToHost, m->s));
+  HIPCHK(hipStreamSynchronize(m->s));
   return 0;
 }
 
-// Host batch -> device X (bf16, padded) and Y; returns padded P
-static int upload_batch(usg_mlp *m, const float *x, const float *y, int n, int *Pout) {
-  const int P = round_up(std::max(n, 1), 128);
-  int rc = ensure_cap(m, P);
-  if (rc) return rc;
-  const int K0 = m->L[0].K, nin = m->d.nin, nout = m->d.nout;
-  std::vector<bf16> X((size_t)P * K0, 0), Xb((size_t)P * K0, 0);
-  for (int p = 0; p < n; p++)
-    for (int k = 0; k < nin; k++) {
-      const bf16 h = to_bf16(x[(size_t)p * nin + k]);
-      X[(size_t)p * K0 + k] = h;
-      Xb[((size_t)(p / 8) * K0 + k) * 8 + p % 8] = h;
-    }
-  HIPCHK(hipMemcpyAsync(m->X, X.data(), X.size() * 2, hipMemcpyHostToDevice, m->s));
-  HIPCHK(hipMemcpyAsync(m->Xb, Xb.data(), Xb.size() * 2, hipMemcpyHostToDevice, m->s));
-  if (y) {
-    std::vector<float> Y((size_t)P * nout, 0.0f);
-    std::memcpy(Y.data(), y, (size_t)n * nout * 4);
-    HIPCHK(hipMemcpyAsync(m->Y, Y.data(), Y.size() * 4, hipMemcpyHostToDevice, m->s));
-  }
-  *Pout = P;
+// The caller's rows on the device.
+static int upload_points(usg_mlp *m, const float *x, const float *y, int n, Points &pt) {
+  const size_t bx = (size_t)n * m->d.nin * sizeof(float), by = (size_t)n * m->d.nout * sizeof(float);
+  int rc = grow(m, m->x, bx);
+  if (rc || (rc = grow(m, m->y, by))) return rc;
+  HIPCHK(hipMemcpyAsync(m->x.p, x, bx, hipMemcpyHostToDevice, m->s));
+  if (y) HIPCHK(hipMemcpyAsync(m->y.p, y, by, hipMemcpyHostToDevice, m->s));
+  pt = Points{nullptr, nullptr, nullptr, (const float *)m->x.p, y ? (const float *)m->y.p : nullptr, n};
   return 0;
 }
 
 int usg_mlp_predict(usg_mlp *m, const float *x, long n, float *y) {
   if (!m || !x || !y || n < 0) return fail(-1, "bad argument");
-  const int step = 65536;
-  const int No = m->L.back().N, nout = m->d.nout;
-  std::vector<float> o;
+  const int step = 262144;  // bounds the device copies of x and y
+  const int nout = m->d.nout;
   for (long a = 0; a < n; a += step) {
     const int cnt = (int)std::min<long>(step, n - a);
-    int P = 0;
-    int rc = upload_batch(m, x + a * m->d.nin, nullptr, cnt, &P);
-    if (rc) return rc;
-    forward(m, P, false);
+    Points pt;
+    if (int rc = upload_points(m, x + a * m->d.nin, nullptr, cnt, pt)) return rc;
+    net(m, false, (cnt + kTile - 1) / kTile, pt, (float *)m->y.p, nullptr);
     HIPCHK(hipGetLastError());
-    o.resize((size_t)P * No);
-    HIPCHK(hipMemcpyAsync(o.data(), m->Z.back(), o.size() * 4, hipMemcpyDeviceToHost, m->s));
-    HIPCHK(hipStreamSynchronize(m->s));
-    for (int p = 0; p < cnt; p++)
-      for (int j = 0; j < nout; j++) y[(a + p) * nout + j] = o[(size_t)p * No + j];
+    HIPCHK(hipMemcpyAsync(y + a * nout, m->y.p, (size_t)cnt * nout * sizeof(float), hipMemcpyDeviceToHost, m->s));
   }
-  return 0;
-}
-
-// loss + output gradient + backward of the batch in X/Y (nv valid of P);
-// with lossbuf, the batch loss goes to lossbuf[slot] on the device (no sync)
-static int loss_and_grads(usg_mlp *m, int P, int nv, float *loss, float *lossbuf = nullptr, int slot = 0,
-                          const AdamStep *adam = nullptr) {
-  forward(m, P, true);
-  const int No = m->L.back().N;
-  const int nbl = P * No / 256;
-  hipLaunchKernelGGL(k_loss, dim3(nbl), dim3(256), 0, m->s, m->Z.back(), No, m->Y, m->d.nout, nv, m->dA, m->dAb,
-                     m->lossp);
-  if (lossbuf)
-    hipLaunchKernelGGL(k_sum_small, dim3(1), dim3(256), 0, m->s, m->lossp, nbl,
-                       (float)(1.0 / ((double)nv * m->d.nout)), lossbuf, slot);
-  backward(m, P, adam);
-  HIPCHK(hipGetLastError());
-  if (loss) {
-    std::vector<float> lp(nbl);
-    HIPCHK(hipMemcpyAsync(lp.data(), m->lossp, nbl * 4, hipMemcpyDeviceToHost, m->s));
-    HIPCHK(hipStreamSynchronize(m->s));
-    double s = 0;
-    for (float v : lp) s += v;
-    *loss = (float)(s / ((double)nv * m->d.nout));
-  }
+  HIPCHK(hipStreamSynchronize(m->s));
   return 0;
 }
 
 int usg_mlp_gradients(usg_mlp *m, const float *x, const float *y, int n, float *loss, float *dw, float *db) {
   if (!m || !x || !y || n <= 0) return fail(-1, "bad argument");
-  int P = 0;
-  int rc = upload_batch(m, x, y, n, &P);
-  if (rc) return rc;
-  rc = loss_and_grads(m, P, n, loss);
-  if (rc) return rc;
-  long ow = 0, ob = 0;
-  for (Layer &L : m->L) {
-    std::vector<float> g((size_t)L.K * L.N), gb(L.N);
-    HIPCHK(hipMemcpyAsync(g.data(), L.gw, g.size() * 4, hipMemcpyDeviceToHost, m->s));
-    HIPCHK(hipMemcpyAsync(gb.data(), L.gb, gb.size() * 4, hipMemcpyDeviceToHost, m->s));
-    HIPCHK(hipStreamSynchronize(m->s));
-    if (dw)
-      for (int k = 0; k < L.k; k++)
-        for (int j = 0; j < L.n; j++) dw[ow + (long)k * L.n + j] = g[(size_t)k * L.N + j];
-    if (db)
-      for (int j = 0; j < L.n; j++) db[ob + j] = gb[j];
-    ow += (long)L.k * L.n;
-    ob += L.n;
+  const int P = round_up(n, 128), nbl = P / 8;
+  int rc = ensure_cap(m, P);
+  if (rc || (rc = grow(m, m->lossp, nbl * sizeof(float))) || (rc = grow(m, m->g, (m->nw + m->nb) * sizeof(float))))
+    return rc;
+  Points pt;
+  if ((rc = upload_points(m, x, y, n, pt))) return rc;
+  float *gw = (float *)m->g.p, *gb = gw + m->nw;
+  net(m, true, P / kTile, pt, nullptr, (float *)m->lossp.p);
+  hipLaunchKernelGGL((k_weights<false>), dim3(m->ntiles), dim3(128), 0, m->s, m->net, m->d_tiles, AdamStep{},
+                     Moments{}, gw, gb);
+  HIPCHK(hipGetLastError());
+  std::vector<float> lp(loss ? nbl : 0);
+  if (loss) HIPCHK(hipMemcpyAsync(lp.data(), m->lossp.p, nbl * sizeof(float), hipMemcpyDeviceToHost, m->s));
+  if (dw) HIPCHK(hipMemcpyAsync(dw, gw, m->nw * sizeof(float), hipMemcpyDeviceToHost, m->s));
+  if (db) HIPCHK(hipMemcpyAsync(db, gb, m->nb * sizeof(float), hipMemcpyDeviceToHost, m->s));
+  HIPCHK(hipStreamSynchronize(m->s));
+  if (loss) {
+    double s = 0;
+    for (float v : lp) s += v;
+    *loss = (float)(s / ((double)n * m->d.nout));
   }
   return 0;
 }
@@ -765,7 +876,7 @@ int usg_mlp_set_data(usg_mlp *m, const float *x, const float *y, long n) {
     m->xs = nullptr;
     m->ys = nullptr;
   }
-  const int K0 = m->L[0].K, nin = m->d.nin, nout = m->d.nout;
+  const int K0 = m->net.K0, nin = m->d.nin, nout = m->d.nout;
   std::vector<bf16> X((size_t)n * K0, 0);
   for (long p = 0; p < n; p++)
     for (int k = 0; k < nin; k++) X[(size_t)p * K0 + k] = to_bf16(x[(size_t)p * nin + k]);
@@ -783,42 +894,34 @@ int usg_mlp_train_epoch(usg_mlp *m, const int *perm, long n, int batch, float lr
   if (n != m->nset) return fail(-1, "perm length differs from the training set");
   for (long i = 0; i < n; i++)
     if (perm[i] < 0 || perm[i] >= n) return fail(-1, "perm entry out of range");
-  const int P = round_up(batch, 128);
-  int rc = ensure_cap(m, P);
-  if (rc) return rc;
-  if (m->idx_cap < n) {
-    if (m->idx) hipFree(m->idx);
-    m->idx = nullptr;
-    HIPCHK(hipMalloc(&m->idx, n * sizeof(int)));
-    m->idx_cap = n;
-  }
-  HIPCHK(hipMemcpyAsync(m->idx, perm, n * sizeof(int), hipMemcpyHostToDevice, m->s));
-  const int K0 = m->L[0].K;
+  const int P = round_up(batch, 128), nbl = P / 8;
   const long nsteps = (n + batch - 1) / batch;
-  if (m->lossbuf_cap < nsteps) {
-    if (m->lossbuf) hipFree(m->lossbuf);
-    m->lossbuf = nullptr;
-    HIPCHK(hipMalloc(&m->lossbuf, nsteps * sizeof(float)));
-    m->lossbuf_cap = nsteps;
-  }
-  long nb = 0;
-  for (long a = 0; a < n; a += batch) {
-    const int nv = (int)std::min<long>(batch, n - a);
-    hipLaunchKernelGGL(k_gather, dim3((unsigned)(((long)P * K0 + 255) / 256)), dim3(256), 0, m->s, m->xs, K0, m->ys,
-                       m->d.nout, m->idx + a, nv, P, m->X, m->Xb, m->Y);
+  int rc = ensure_cap(m, P);
+  if (rc || (rc = grow(m, m->idx, n * sizeof(int))) || (rc = grow(m, m->lossp, (size_t)nsteps * nbl * sizeof(float))) ||
+      (rc = grow(m, m->losses, nsteps * sizeof(float))))
+    return rc;
+  HIPCHK(hipMemcpyAsync(m->idx.p, perm, n * sizeof(int), hipMemcpyHostToDevice, m->s));
+  float *lossp = (float *)m->lossp.p;
+  int nv = 0;
+  for (long q = 0; q < nsteps; q++) {
+    nv = (int)std::min<long>(batch, n - q * batch);
+    net(m, true, P / kTile, Points{m->xs, m->ys, (const int *)m->idx.p + q * batch, nullptr, nullptr, nv}, nullptr,
+        lossp + q * nbl);
     m->step++;
     const AdamStep st{lr, 1.0f - std::pow(0.9f, (float)m->step), 1.0f - std::pow(0.999f, (float)m->step)};
-    rc = loss_and_grads(m, P, nv, nullptr, m->lossbuf, (int)nb, &st);
-    if (rc) return rc;
-    nb++;
+    hipLaunchKernelGGL((k_weights<true>), dim3(m->ntiles), dim3(128), 0, m->s, m->net, m->d_tiles, st, m->mo, nullptr,
+                       nullptr);
   }
+  hipLaunchKernelGGL(k_losses, dim3((unsigned)nsteps), dim3(256), 0, m->s, lossp, nbl,
+                     (float)(1.0 / ((double)batch * m->d.nout)), (float)(1.0 / ((double)nv * m->d.nout)),
+                     (float *)m->losses.p);
   HIPCHK(hipGetLastError());
-  std::vector<float> lb(nb);
-  HIPCHK(hipMemcpyAsync(lb.data(), m->lossbuf, nb * sizeof(float), hipMemcpyDeviceToHost, m->s));
+  std::vector<float> lb(nsteps);
+  HIPCHK(hipMemcpyAsync(lb.data(), m->losses.p, nsteps * sizeof(float), hipMemcpyDeviceToHost, m->s));
   HIPCHK(hipStreamSynchronize(m->s));
   double lsum = 0;
   for (float v : lb) lsum += v;
-  if (loss_out) *loss_out = (float)(lsum / std::max<long>(nb, 1));
+  if (loss_out) *loss_out = (float)(lsum / nsteps);
   return 0;
 }
 
