@@ -428,11 +428,11 @@ class Solver:
     def field(self, fid: int) -> np.ndarray:
         if fid == F_UEDGE:
             nf = sum(m.nf for m in self.meshes)
-            out = np.zeros(nf * 4)
+            out = np.empty(nf * 4)
             _check(lib().usg_get_field(self._h, fid, out.ctypes.data_as(_dp), out.size))
             return out.reshape(nf, 4)
         w = _FIELD_WIDTH[fid]
-        out = np.zeros(self.nc * w)
+        out = np.empty(self.nc * w)
         _check(lib().usg_get_field(self._h, fid, out.ctypes.data_as(_dp), out.size))
         return out.reshape(self.nc, w) if w > 1 else out
 
