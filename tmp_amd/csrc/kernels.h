@@ -76,9 +76,8 @@ struct DevMesh {
   // 0 hole, -1 receptor.  Only field cells are updated by the sweeps and
   // enter the residual norm; receptors are set from their donors.
   const signed char *blank;
-  // boundary faces: bface[nbf] (ascending), and each face's index in that
-  // list (bidx[f], -1 for an interior face)
-  const int *bface, *bidx;
+  // each face's index among the nbf boundary faces (-1 for an interior face)
+  const int *bidx;
   int nbf;
 };
 
@@ -115,8 +114,8 @@ struct DevState {
   // dual time stepping: the conservative state at the two previous
   // physical time levels, W^n and W^(n-1) ([2][nc][2]; null when off)
   double *Wt1, *Wt2;
-  // face states of the boundary faces for the gradient kernel, [4][nbf]
-  // (k_bstate at the start of every residual)
+  // face states of the boundary faces, from and for the gradient kernel,
+  // [2][nbf][2] (pidx)
   double *Ub;
   // FP32 storage of the mixed-precision mode (null in FP64 mode, where the
   // double arrays above hold these quantities)

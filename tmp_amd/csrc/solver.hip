@@ -82,35 +82,6 @@ __device__ __forceinline__ bool get_slot(const DevMesh &m, int s, int c, Slot &o
   return true;
 }
 
-// ---------------------------------------------------------------------------
-// k_bstate: the face state of every boundary face (BoundaryStrategy::
-// HandleInvicidBoundary / HandleViscousBoundary, BoundaryStrategy.h:73-335)
-// from its cell's current state, for the gradient kernel, which would
-// otherwise hold the far-field Riemann state's registers (50 VGPRs, one
-// wave per SIMD) for the few cells that have a boundary face.  The slip-wall
-// check is counted here.
-// ---------------------------------------------------------------------------
-template <bool VISC, bool B>
-__global__ __launch_bounds__(kBlock) void k_bstate(const DevMesh m, const DevState s, const Consts k_) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= m.nbf) return;
-  const int f = m.bface[b], c = m.flc[f], nc = m.nc;
-  const Consts k = case_consts<B>(m, k_, c);
-  double Ul[4], Ue[4];
-  load4p(s.U, nc, c, Ul);
-  if (!boundary_state<VISC>(k, m.frc[f], Ul, m.fnx[f], m.fny[f], Ue)) {
-    atomicAdd(&s.err[1], 1);
-    if constexpr (B) atomicOr(&s.err[2 + m.ccase[c]], 2);
-  }
-  for (int j = 0; j < 4; j++) s.Ub[(size_t)j * m.nbf + b] = Ue[j];
-}
-
-// ---------------------------------------------------------------------------
-// k_grad: boundary states + gradients + limiter (+ SST F1/F2)
-// Euler2D::updateEdgeValues/solveGradient (Euler2D.cpp:202-240),
-// ViscousFlow2D.cpp:174-252, Vankatakrishnan_Limiter.hpp:69-200,
-// LaminarFluxStrategy::computeMu (cells), SSTKWStrategy.h:616-722.
-// ---------------------------------------------------------------------------
 // Mesh arrays by compute type.
 template <typename T>
 __device__ __forceinline__ const T *fnx_of(const DevMesh &m) { return pickc<T>(m.fnx, m.fnxf); }
@@ -190,9 +161,41 @@ __global__ __launch_bounds__(kBlock) void k_grad(const DevMesh m, const DevState
   for (int i = 0; i < 4; i++) nb[i] = m.cnb[i * nc + c];
   const bool four = fe[3] != kNoSlot;
   if (!four) nb[3] = c;
+  // The face states of the cell's boundary faces (BoundaryStrategy::
+  // HandleInvicidBoundary / HandleViscousBoundary, BoundaryStrategy.h:73-335)
+  // go to memory and come back with the gathers: the far-field Riemann state
+  // takes registers only while nothing else does (116 -> 117 VGPRs laminar).
+  // A launch of its own for them, one thread per boundary face, was 4.5 us of
+  // mostly launch.  Measured with it, per residual: Euler 20 k cells 6.5 + 4.6
+  // -> 8.2 us, 106 k 12.9 + 4.5 -> 13.7 us; SST 1 M 109 + 5.9 -> 104 us.  The
+  // slip-wall check is counted here.
+  int at[4], todo = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    at[i] = nb[i];
+    todo |= nb[i] < 0 ? 1 << i : 0;
+  }
+  while (todo) {
+    const int q = __builtin_ctz(todo);
+    todo &= todo - 1;
+    const int f = q == 0 ? fe[0] : q == 1 ? fe[1] : q == 2 ? fe[2] : fe[3];
+    const int bc = q == 0 ? nb[0] : q == 1 ? nb[1] : q == 2 ? nb[2] : nb[3];
+    double Ub[4];
+    if (!boundary_state<F::visc>(k, bc, Ucd, m.fnx[f], m.fny[f], Ub)) {
+      atomicAdd(&s.err[1], 1);
+      if constexpr (B) atomicOr(&s.err[2 + m.ccase[c]], 2);
+    }
+    const int b = m.bidx[f];
+    store4p(s.Ub, m.nbf, b, Ub);
+#pragma unroll
+    for (int i = 0; i < 4; i++) at[i] = i == q ? b : at[i];
+  }
   double Unbd[4][4], tnb[4][2];
 #pragma unroll
-  for (int i = 0; i < 4; i++) load4p(s.U, nc, nb[i] >= 0 ? nb[i] : c, Unbd[i]);
+  for (int i = 0; i < 4; i++) {
+    const bool in = nb[i] >= 0;
+    load4p(in ? s.U : s.Ub, in ? nc : m.nbf, at[i], Unbd[i]);
+  }
   if (F::sst) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -241,10 +244,10 @@ __global__ __launch_bounds__(kBlock) void k_grad(const DevMesh m, const DevState
         }
       }
     } else {
-      // the face state k_bstate formed for this residual
-      const int b = m.bidx[f];
-      for (int j = 0; j < 4; j++) Ued[j] = s.Ub[(size_t)j * m.nbf + b];
-      for (int j = 0; j < 4; j++) Ue[j] = kDiff ? T(Ued[j] - Ucd[j]) : T(Ued[j]);
+      for (int j = 0; j < 4; j++) {
+        Ued[j] = Unbd[i][j];
+        Ue[j] = kDiff ? T(Ued[j] - Ucd[j]) : T(Ued[j]);
+      }
     }
     // Green-Gauss: + for the left cell, - for the right cell (x - y and
     // x + (-y) are the same bits)
@@ -2276,9 +2279,6 @@ template <int FLOW, typename T, bool B>
 static void launch_residual(usg_ctx *c, hipEvent_t ea, hipEvent_t eb) {
   const XSlice cs = slice(c->hm.cell_off.data()), fs = slice(c->hm.face_off.data());
   const int bg = c->blk[USG_K_GRAD], bf = c->blk[USG_K_FACE], bc = c->blk[USG_K_CELL];
-  if (c->dm.nbf > 0)
-    hipLaunchKernelGGL((k_bstate<Flow<FLOW>::visc, B>), dim3(grid(c->dm.nbf)), dim3(kBlock), 0, c->stream, c->dm,
-                       c->ds, c->k);
   hipLaunchKernelGGL((k_grad<FLOW, T, B>), dim3(xgrid(cs, bg)), dim3(bg), 0, c->stream, c->dm, c->ds, c->k,
                      c->d_cell_list, cs);
   if constexpr (std::is_same<T, double>::value) {
@@ -2971,17 +2971,13 @@ static int ctx_setup(usg_ctx *c, usg_ctx **out) {
   CK(upload(c, &c->d_cell_list, h.cell_list.data(), nc));
   CK(upload(c, &c->d_face_list, h.face_list.data(), nf));
   {
-    // boundary faces for k_bstate, and each face's index among them
-    std::vector<int> bface, bidx(nf, -1);
+    // each boundary face's index among them (k_grad)
+    std::vector<int> bidx(nf, -1);
+    dm.nbf = 0;
     for (int f = 0; f < nf; f++)
-      if (h.frc[f] < 0) {
-        bidx[f] = (int)bface.size();
-        bface.push_back(f);
-      }
-    dm.nbf = (int)bface.size();
-    CK(upload(c, (int **)&dm.bface, bface.data(), std::max<size_t>(bface.size(), 1)));
+      if (h.frc[f] < 0) bidx[f] = dm.nbf++;
     CK(upload(c, (int **)&dm.bidx, bidx.data(), nf));
-    CK(dalloc(c, &c->ds.Ub, 4 * std::max<size_t>(bface.size(), 1)));
+    CK(dalloc(c, &c->ds.Ub, 4 * std::max<size_t>(dm.nbf, 1)));
   }
   std::vector<int> wc(h.wall_faces.size());
   for (size_t i = 0; i < wc.size(); i++) wc[i] = h.flc[h.wall_faces[i]];
