@@ -1094,15 +1094,15 @@ __device__ void norm_partial_block(const DevMesh &m, const double *R, const int 
 __device__ void norm_ring_block(const double *partial, const int *boff, double *ring, int cap, int *ctr, int cs,
                                 int ncase);
 
-// Residual-norm blocks appended to a sweep launch of a single case with
-// kBlock-thread blocks: launch blocks [nsweep, nsweep + n) run the norm's
-// per-block partial sums (kind 1: n = one per norm block) or its ring sum
-// (kind 2: n = 1), the same code on the same cells as k_norm_partial and
-// k_norm_ring, which they replace.  R is not written by the sweeps, and the
-// ring sum runs in the sweep launch after the partial sums (forward or
-// backward).
+// Residual-norm blocks appended to a sweep launch with kBlock-thread blocks:
+// launch blocks [nsweep, nsweep + n) run the norm's per-block partial sums
+// (kind 1: n = one per norm block) or its ring sums (kind 2: n = one per
+// case), the same code on the same cells as k_norm_partial and k_norm_ring,
+// which they replace.  R is not written by the sweeps, and the ring sum runs
+// in the sweep launch after the partial sums (forward or backward).  Three
+// launches of their own cost a batch of 8 x 12 k cells 8 of 97 us an iteration.
 struct NormBlocks {
-  int kind = 0, nsweep = 0, cap = 0;
+  int kind = 0, nsweep = 0, cap = 0, ncase = 1;
   const double *R = nullptr;
   const int *b0 = nullptr, *b1 = nullptr, *boff = nullptr;
   double *partial = nullptr, *ring = nullptr;
@@ -1319,7 +1319,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     if (nb.kind == 1)
       norm_partial_block(m, nb.R, nb.b0, nb.b1, nb.partial, (int)blockIdx.x - nb.nsweep);
     else
-      norm_ring_block(nb.partial, nb.boff, nb.ring, nb.cap, nb.ctr, 0, 1);
+      norm_ring_block(nb.partial, nb.boff, nb.ring, nb.cap, nb.ctr, (int)blockIdx.x - nb.nsweep, nb.ncase);
     return;
   }
   if ((int)blockIdx.x < tl.nblk) {
@@ -1649,7 +1649,7 @@ template <int FLOW, typename T, bool B>
 __global__ __launch_bounds__(kBlock) void k_level_finish(const DevMesh m, const DevState s, const Consts k_,
                                                          const LevelView v, const NormBlocks nbk) {
   if (nbk.kind && (int)blockIdx.x >= nbk.nsweep) {
-    norm_ring_block(nbk.partial, nbk.boff, nbk.ring, nbk.cap, nbk.ctr, 0, 1);
+    norm_ring_block(nbk.partial, nbk.boff, nbk.ring, nbk.cap, nbk.ctr, (int)blockIdx.x - nbk.nsweep, nbk.ncase);
     return;
   }
   const int c = blockIdx.x * blockDim.x + threadIdx.x, nc = m.nc;
@@ -1765,24 +1765,20 @@ __global__ __launch_bounds__(kBlock) void k_norm_final(const double *partial, co
   double v = case_sum(partial, boff, blockIdx.x);
   if (threadIdx.x == 0) out[blockIdx.x] = sqrt(v);
 }
-// one block per case: ring[(ctr % cap) * ncase + case] = sqrt(sum); the
-// counter is advanced by this kernel when there is one case, else by
-// k_add_int launched after it (no block may see another's increment)
+// one block per case: ring[(ctr[case] % cap) * ncase + case] = sqrt(sum), and
+// the case's counter goes on
 __device__ void norm_ring_block(const double *partial, const int *boff, double *ring, int cap, int *ctr, int cs,
                                 int ncase) {
   double v = case_sum(partial, boff, cs);
   if (threadIdx.x == 0) {
-    int i = *ctr;
+    const int i = ctr[cs];
     ring[(size_t)(i % cap) * ncase + cs] = sqrt(v);
-    if (ncase == 1) *ctr = i + 1;
+    ctr[cs] = i + 1;
   }
 }
 __global__ __launch_bounds__(kBlock) void k_norm_ring(const double *partial, const int *boff, double *ring,
                                                       int cap, int *ctr) {
   norm_ring_block(partial, boff, ring, cap, ctr, blockIdx.x, gridDim.x);
-}
-__global__ void k_add_int(int *p, int v) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *p = *p + v;
 }
 // Fields between their device layouts (paired, pidx, or one array per
 // component) and rows of 1 << lv values in pinned host memory, which the
@@ -1808,8 +1804,9 @@ __global__ __launch_bounds__(kBlock) void k_from_host(const double *__restrict__
 __global__ void k_err_host(const int *err, int *out) {
   if (threadIdx.x < 2) out[threadIdx.x] = err[threadIdx.x];
 }
-__global__ void k_set_int(int *p, int v) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
+__global__ __launch_bounds__(kBlock) void k_set_int(int *p, int n, int v) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) p[i] = v;
 }
 
 // Viscous momentum flux tau . n A of wall face f of its cell c, from the
@@ -2544,6 +2541,7 @@ static void launch_level_sweeps(usg_ctx *c, bool fuse_norm) {
     nb.partial = c->d_partial;
     nb.ring = c->d_ring;
     nb.ctr = c->d_ctr;
+    nb.ncase = c->ncase;
     nb2 = nb;
     nb2.kind = 2;
   }
@@ -2555,13 +2553,13 @@ static void launch_level_sweeps(usg_ctx *c, bool fuse_norm) {
   for (int w = 1; w < c->level_from[1]; w++) launch_wave<FLOW, false, T, B>(c, w, none, 0, SweepTail{});
   hipLaunchKernelGGL((k_levels<FLOW, false>), dim3(c->ncase), dim3(kLevelThreads), c->level_lds, c->stream, c->ds,
                      c->lv, c->hm.nc);
-  hipLaunchKernelGGL((k_level_finish<FLOW, T, B>), dim3(c->nblk + (fuse_norm ? 1 : 0)), dim3(kBlock), 0, c->stream,
+  hipLaunchKernelGGL((k_level_finish<FLOW, T, B>), dim3(c->nblk + (fuse_norm ? c->ncase : 0)), dim3(kBlock), 0, c->stream,
                      c->dm, c->ds, c->k, c->lv, nb2);
 }
 
 // With fuse_norm, the first two sweep launches of the iteration also carry
 // the residual norm into the ring (NormBlocks): the partial sums on the
-// first, the ring sum on the second (forward or backward: neither writes R).
+// first, the ring sums on the second (forward or backward: neither writes R).
 template <int FLOW, typename T, bool B>
 static void launch_sweeps(usg_ctx *c, bool fuse_norm) {
   if (c->levels) {
@@ -2585,7 +2583,8 @@ static void launch_sweeps(usg_ctx *c, bool fuse_norm) {
       nb.partial = c->d_partial;
       nb.ring = c->d_ring;
       nb.ctr = c->d_ctr;
-      extra = nb.kind == 1 ? c->nnb : 1;
+      nb.ncase = c->ncase;
+      extra = nb.kind == 1 ? c->nnb : c->ncase;
     }
     launch++;
     return nb;
@@ -3108,7 +3107,7 @@ static int ctx_setup(usg_ctx *c, usg_ctx **out) {
   CK(dalloc(c, &c->d_force, 2 * (size_t)c->ncase));
   CK(ensure_norms(c, 16 * c->ncase));
   CK(dalloc(c, &c->d_ring, (size_t)kRing * c->ncase));
-  CK(dalloc(c, &c->d_ctr, 1));
+  CK(dalloc(c, &c->d_ctr, c->ncase));
   CK(make_stage(c));
   CK(build_levels(c));
 #undef CK
@@ -3213,13 +3212,12 @@ static void launch_norm_ring(usg_ctx *c) {
                      c->d_partial);
   hipLaunchKernelGGL(k_norm_ring, dim3(c->ncase), dim3(kBlock), 0, c->stream, c->d_partial, c->d_nboff, c->d_ring,
                      kRing, c->d_ctr);
-  if (c->ncase > 1) hipLaunchKernelGGL(k_add_int, dim3(1), dim3(64), 0, c->stream, c->d_ctr, 1);
 }
 
-// The norm rides on the sweep launches for a single case whose sweeps use
-// kBlock-thread blocks and make at least two launches.
+// The norm rides on the sweep launches if these use kBlock-thread blocks and
+// there are at least two.
 static bool fuse_norm(const usg_ctx *c) {
-  return c->ncase == 1 && (c->levels || (c->blk[USG_K_SWEEP] == kBlock && sweep_launches(c) >= 2));
+  return c->levels || (c->blk[USG_K_SWEEP] == kBlock && sweep_launches(c) >= 2);
 }
 
 // One LU-SGS iteration (LUSGSIntegrator::UpdateSerial): residual, norm into
@@ -3291,7 +3289,7 @@ static bool ensure_graphs(usg_ctx *c) {
 
 int usg_lusgs_step(usg_ctx *c, int n, double *res_hist) {
   if (!c || n < 0) return fail(USG_ERR_ARG, "bad argument");
-  hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, c->stream, c->d_ctr, 0);
+  hipLaunchKernelGGL(k_set_int, dim3(grid(c->ncase)), dim3(kBlock), 0, c->stream, c->d_ctr, c->ncase, 0);
   int done = 0;
   while (done < n) {
     const int chunk = std::min(n - done, kRing);
@@ -3317,7 +3315,7 @@ int usg_lusgs_step(usg_ctx *c, int n, double *res_hist) {
     if (res_hist)
       HIPCHK(hipMemcpyAsync(res_hist + (size_t)done * c->ncase, c->d_ring, (size_t)chunk * c->ncase * sizeof(double),
                             hipMemcpyDeviceToHost, c->stream));
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, c->stream, c->d_ctr, 0);
+    hipLaunchKernelGGL(k_set_int, dim3(grid(c->ncase)), dim3(kBlock), 0, c->stream, c->d_ctr, c->ncase, 0);
     done += chunk;
   }
   c->have_residual = false;
