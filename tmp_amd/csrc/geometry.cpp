@@ -178,8 +178,29 @@ void by_part(const std::vector<int> &items, const std::vector<int> &item_part, s
   for (int it : items) out[pos[item_part[it]]++] = it;
 }
 
+// The chunk lists, from cell_list (of one mesh or of a union).
+void chunk_lists(HostMesh &m) {
+  std::vector<int> pos(m.nc);
+  for (int i = 0; i < m.nc; i++) pos[m.cell_list[i]] = i;
+  auto build = [&](int n, auto cell_of, std::vector<int> &list, std::vector<int> &off) {
+    const int k = (n + kChunkItems - 1) / kChunkItems;
+    std::vector<std::pair<int, int>> key(k);
+    for (int i = 0; i < k; i++) key[i] = {pos[cell_of(std::min(n - 1, i * kChunkItems + kChunkItems / 2))], i};
+    std::sort(key.begin(), key.end());
+    list.resize(k);
+    off.assign(kParts + 1, k);
+    int i = 0;
+    for (int p = 0; p < kParts; p++) {
+      off[p] = i;
+      for (; i < k && key[i].first < m.cell_off[p + 1]; i++) list[i] = key[i].second;
+    }
+  };
+  build(m.nc, [](int c) { return c; }, m.cell_chunks, m.cell_chunk_off);
+  build(m.nf, [&](int f) { return m.flc[f]; }, m.face_chunks, m.face_chunk_off);
+}
+
 void xcd_lists(HostMesh &m) {
-  const int nc = m.nc, nf = m.nf;
+  const int nc = m.nc;
   double xmin = 1e300, xmax = -1e300, ymin = 1e300, ymax = -1e300;
   for (int i = 0; i < nc; i++) {
     xmin = std::min(xmin, m.cc[2 * i]);
@@ -206,13 +227,7 @@ void xcd_lists(HostMesh &m) {
   for (int r = 0; r < nc; r++) all[r] = key[r].second;
   m.cell_off.assign(kParts + 1, 0);
   by_part(all, m.part, m.cell_list, m.cell_off.data());
-  std::vector<int> fpart(nf), fall(nf);
-  for (int f = 0; f < nf; f++) {
-    fpart[f] = m.part[m.flc[f]];
-    fall[f] = f;
-  }
-  m.face_off.assign(kParts + 1, 0);
-  by_part(fall, fpart, m.face_list, m.face_off.data());
+  chunk_lists(m);
   auto waves_by_part = [&](const std::vector<int> &cells, const std::vector<int> &woff, std::vector<int> &list,
                            std::vector<int> &poff) {
     const int nw = (int)woff.size() - 1;
@@ -426,9 +441,7 @@ void merge_meshes(const std::vector<HostMesh> &cases, HostMesh &u) {
   merge_parts([](const HostMesh &c) -> const std::vector<int> & { return c.cell_list; },
               [](const HostMesh &c) -> const std::vector<int> & { return c.cell_off; }, u.case_cell, u.cell_list,
               u.cell_off);
-  merge_parts([](const HostMesh &c) -> const std::vector<int> & { return c.face_list; },
-              [](const HostMesh &c) -> const std::vector<int> & { return c.face_off; }, u.case_face, u.face_list,
-              u.face_off);
+  chunk_lists(u);
   // waves: wave w, part p of the union = the cases' (w, p) slices in case order
   auto merge_waves = [&](bool fwd, std::vector<int> &list, std::vector<int> &poff) {
     int nw = 0;

@@ -34,14 +34,15 @@ struct HostMesh {
   bool use_ranges = false;
   std::vector<int> wall_faces;
   // XCD-aware work lists: cells / faces / wave cells grouped by spatial part
-  // (kParts equal slices of the Hilbert curve of the cell centres; a face
-  // belongs to its left cell's part); cells in Hilbert order, faces and wave
-  // cells in ascending id inside a part.  Launches
+  // (kParts equal slices of the Hilbert curve of the cell centres); cells in
+  // Hilbert order, wave cells in ascending id inside a part.  Launches
   // send part p's blocks to XCD p (blockIdx % kParts) so that neighbour
   // gathers hit the XCD's own L2.
   std::vector<int> part;                      // [nc]
   std::vector<int> cell_list, cell_off;       // [nc], [kParts+1]
-  std::vector<int> face_list, face_off;       // [nf], [kParts+1]
+  // aligned chunks of kChunkItems consecutive cells (faces), in the Hilbert
+  // order and the part of their middle cell (its middle face's left cell)
+  std::vector<int> cell_chunks, cell_chunk_off, face_chunks, face_chunk_off;
   std::vector<int> fwd_list, fwd_poff;        // [nc], [nwaves*(kParts+1)]
   std::vector<int> bwd_list, bwd_poff;        // [nc], [nwaves*(kParts+1)]
   // batch of independent cases (one case when built by build_mesh): case i
@@ -50,7 +51,8 @@ struct HostMesh {
   std::vector<int> case_cell, case_face, case_wall;
 };
 
-constexpr int kParts = 8;  // XCDs of an MI355X
+constexpr int kParts = 8;        // XCDs of an MI355X
+constexpr int kChunkItems = 64;  // a wave's
 
 // Validates the faces and returns each cell's vertices in the reference's
 // order (Brick4Cobalt2D::insert, CellBrick.cpp:13-136): cnode[nc*4] (-1

@@ -30,6 +30,18 @@ __device__ __forceinline__ bool xcd_item_at(const int *__restrict__ items, const
 __device__ __forceinline__ bool xcd_item(const int *__restrict__ items, const XSlice &sl, int &item) {
   return xcd_item_at(items, sl, (int)blockIdx.x, item);
 }
+// The same with a list of chunks of kWaveItems items, one per wave, of n items
+// in all: a wave's own items are consecutive, its neighbours in time are its
+// neighbours in space.
+constexpr int kWaveItems = 64;
+__device__ __forceinline__ bool xcd_chunk(const int *__restrict__ chunks, const XSlice &sl, int n, int &item) {
+  const int b = (int)blockIdx.x, part = b % kXcd;
+  const int t = b / kXcd * (int)blockDim.x + (int)threadIdx.x;
+  const int i = __builtin_amdgcn_readfirstlane(sl.off[part] + t / kWaveItems);
+  if (i >= sl.off[part + 1]) return false;
+  item = chunks[i] * kWaveItems + t % kWaveItems;
+  return item < n;
+}
 constexpr int kWallD = -2;
 constexpr int kFarD = -3;
 
