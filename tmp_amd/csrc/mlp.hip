@@ -234,22 +234,42 @@ __global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Poi
   bf16x8 b[2 * KM];
   load_frags<4>(b, m.wf, K0 / 32, W / 16, 2 * wave);
 
-  // inputs
+  // inputs and targets; every load of a round trip is made before the first is
+  // waited for
+  const int nx = kTile * K0 / 8, ny = kTile * nout;
   if (pt.xs) {
-    for (int i = tid; i < kTile * K0 / 8; i += kThreads) {
-      const int p = i / (K0 / 8), c = i % (K0 / 8) * 8;
-      bf16x8 v = {};
-      if (p0 + p < pt.nv) v = load8(pt.xs + (size_t)pt.idx[p0 + p] * K0 + c);
-      *reinterpret_cast<bf16x8 *>(sx + p * ld0 + c) = v;
+    constexpr int NI = (kTile * 128 / 8 + kThreads - 1) / kThreads;
+    int q[NI], qy = 0;
+#pragma unroll
+    for (int j = 0; j < NI; j++) q[j] = pt.idx[min(p0 + min(tid + j * kThreads, nx - 1) / (K0 / 8), pt.nv - 1)];
+    if (TRAIN) qy = pt.idx[min(p0 + min(tid, ny - 1) / nout, pt.nv - 1)];
+    bf16x8 v[NI];
+#pragma unroll
+    for (int j = 0; j < NI; j++)
+      v[j] = load8(pt.xs + (size_t)q[j] * K0 + min(tid + j * kThreads, nx - 1) % (K0 / 8) * 8);
+    const float y = TRAIN ? pt.ys[(size_t)qy * nout + tid % nout] : 0.0f;
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      const int i = tid + j * kThreads, p = i / (K0 / 8), c = i % (K0 / 8) * 8;
+      if (i < nx) *reinterpret_cast<bf16x8 *>(sx + p * ld0 + c) = p0 + p < pt.nv ? v[j] : bf16x8{};
     }
+    if (TRAIN && tid < ny) sy[tid] = p0 + tid / nout < pt.nv ? y : 0.0f;
   } else {
-    for (int i = tid; i < kTile * K0; i += kThreads) {
-      const int p = i / K0, c = i % K0;
-      sx[p * ld0 + c] = p0 + p < pt.nv && c < nin ? to_bf16(pt.x[(size_t)(p0 + p) * nin + c]) : (bf16)0;
+    constexpr int NI = (kTile * 128 + kThreads - 1) / kThreads;
+    float v[NI];
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      const int i = min(tid + j * kThreads, kTile * K0 - 1);
+      v[j] = pt.x[(size_t)min(p0 + i / K0, pt.nv - 1) * nin + min(i % K0, nin - 1)];
+    }
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      const int i = tid + j * kThreads, p = i / K0, c = i % K0;
+      if (i < kTile * K0) sx[p * ld0 + c] = p0 + p < pt.nv && c < nin ? to_bf16(v[j]) : (bf16)0;
     }
   }
   if (TRAIN)
-    for (int i = tid; i < kTile * nout; i += kThreads) {
+    for (int i = tid + (pt.xs ? kThreads : 0); i < ny; i += kThreads) {
       const int p = p0 + i / nout;
       float v = 0.0f;
       if (p < pt.nv) v = pt.xs ? pt.ys[(size_t)pt.idx[p] * nout + i % nout] : pt.y[(size_t)p0 * nout + i];
