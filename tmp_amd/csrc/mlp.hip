@@ -136,13 +136,22 @@ __device__ __forceinline__ float recip_mid(float x) {
   r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
   return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
 }
-// sigmoid of four values: 16 instructions each where |z| <= 87, against 24 of
-// expf and a division, which take the rest
-__device__ __forceinline__ void sigmoid4(const float (&z)[4], float (&s)[4]) {
-  if (fmaxf(fmaxf(fabsf(z[0]), fabsf(z[1])), fmaxf(fabsf(z[2]), fabsf(z[3]))) <= 87.0f)
-    for (int r = 0; r < 4; r++) s[r] = recip_mid(1.0f + exp_mid(-z[r]));
-  else
-    for (int r = 0; r < 4; r++) s[r] = sigmoid(z[r]);
+// sigmoid of eight values: 16 instructions each where |z| <= 87, against 24 of
+// expf and a division, which the rest take.  sigmoid_mid does the common ones
+// without a branch (matrix instructions can go among them) and says whether
+// they were all.
+__device__ __forceinline__ bool sigmoid_mid(const float (&z)[2][4], float (&s)[2][4]) {
+  float top = 0.0f;
+  for (int t = 0; t < 2; t++)
+    for (int r = 0; r < 4; r++) {
+      s[t][r] = recip_mid(1.0f + exp_mid(-z[t][r]));
+      top = fmaxf(top, fabsf(z[t][r]));
+    }
+  return top <= 87.0f;
+}
+__device__ __forceinline__ void sigmoid_rest(const float (&z)[2][4], float (&s)[2][4]) {
+  for (int t = 0; t < 2; t++)
+    for (int r = 0; r < 4; r++) s[t][r] = sigmoid(z[t][r]);
 }
 typedef bf16 bf16x4u __attribute__((ext_vector_type(4)));
 // four FP32 -> BF16, round to nearest even (as to_bf16)
@@ -169,21 +178,27 @@ __device__ __forceinline__ void load_frags(bf16x8 *b, const bf16 *w, int steps, 
       b[2 * s + t] = load8(w + ((size_t)(min(s, steps - 1) * tiles + tile + t) * 64 + lane) * 8);
 }
 
-// acc[p tile][n tile] of one wave: 32 points x 32 outputs, A rows in LDS
+// acc[n tile] of one wave: 16 points x 32 outputs, A rows in LDS
 template <int T>
-__device__ __forceinline__ void product(floatx4 (&acc)[2][2], const bf16 *a, int lda, const bf16x8 *b, int steps) {
+__device__ __forceinline__ void product(floatx4 (&acc)[2], const bf16 *a, int lda, const bf16x8 *b, int steps) {
   const int lane = threadIdx.x % kWave;
-  for (int i = 0; i < 2; i++)
-    for (int t = 0; t < 2; t++) acc[i][t] = floatx4{0, 0, 0, 0};
+  for (int t = 0; t < 2; t++) acc[t] = floatx4{0, 0, 0, 0};
   const bf16 *r = a + (lane % 16) * lda + (lane / 16) * 8;
 #pragma unroll
   for (int s = 0; s < T; s++) {
     if (s >= steps) continue;
-    const bf16x8 a0 = load8(r + s * 32), a1 = load8(r + 16 * lda + s * 32);
-    for (int t = 0; t < 2; t++) {
-      acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[2 * s + t], acc[0][t], 0, 0, 0);
-      acc[1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[2 * s + t], acc[1][t], 0, 0, 0);
-    }
+    const bf16x8 x = load8(r + s * 32);
+    for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, b[2 * s + t], acc[t], 0, 0, 0);
+  }
+}
+// N matrix instructions among the vector ones around them, one after every 10
+// (a wave's activations of one half are 11 of them per matrix instruction).
+template <int N>
+__device__ __forceinline__ void interleave() {
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x2, 10, 0);
   }
 }
 
@@ -213,7 +228,9 @@ __device__ __forceinline__ void put4(bf16 *rows, int ld, bf16 *op, int p0, int N
 // barriers the rest, and the first loads of the points 12000 of a block's
 // 120000 cycles.  Measured at 8 x 256 on 16384 points: 112 us, against 350 us
 // for a launch per product (and one each for the batch, the loss and the last
-// layer); inference of 12576 points 50 us against 98 us.
+// layer).  Inference of 12576 points takes 36 us, against 98 us, with the two
+// halves of a block's points one behind the other (125 VGPRs: two blocks to a
+// CU; both at once took 179 VGPRs and 45 us).
 // ---------------------------------------------------------------------------
 template <int W, bool TRAIN>
 __global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Points pt, float *__restrict__ out,
@@ -287,25 +304,46 @@ __global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Poi
   }
 
   // forward: hidden layers
-  floatx4 acc[2][2];
   for (int l = 0; l < nl - 1; l++) {
     float bl[2];
     for (int t = 0; t < 2; t++) bl[t] = m.b[l * W + wave * 32 + t * 16 + ln];
-    if (l == 0)
-      product<4>(acc, sx, ld0, b, K0 / 32);
-    else
-      product<KS>(acc, rows(l - 1), ld, b, KS);
-    const bool last = l == nl - 2;  // (of the last layer every wave loads the two n tiles there are)
-    load_frags<KS>(b, m.wf + m.frag(l + 1), KS, last ? kOut / 16 : W / 16, last ? 0 : 2 * wave);
+    const bf16 *in = l == 0 ? sx : rows(l - 1);
     bf16 *h = rows(l), *hb = TRAIN ? m.in + m.inp(l + 1) : nullptr;
-    for (int i = 0; i < 2; i++)
+    const bool last = l == nl - 2;  // (of the last layer every wave loads the two n tiles there are)
+    const bf16 *wn = m.wf + m.frag(l + 1);
+    // the second half's product runs among the first half's activations
+    floatx4 acc[2][2];
+    float z[2][4], s[2][4];
+    auto pre = [&](int i) {
+      for (int t = 0; t < 2; t++)
+        for (int r = 0; r < 4; r++) z[t][r] = acc[i][t][r] + bl[t];
+    };
+    auto put = [&](int i, bool mid) {
+      if (!mid) sigmoid_rest(z, s);
       for (int t = 0; t < 2; t++) {
-        float z[4], s[4];
-        for (int r = 0; r < 4; r++) z[r] = acc[i][t][r] + bl[t];
-        sigmoid4(z, s);
-        for (int r = 0; r < 4; r++) z[r] = z[r] * s[r];
-        put4(h, ld, hb, p0, W, i * 16 + lp, wave * 32 + t * 16 + ln, to_bf16x4(z));
+        float v[4];
+        for (int r = 0; r < 4; r++) v[r] = z[t][r] * s[t][r];
+        put4(h, ld, hb, p0, W, i * 16 + lp, wave * 32 + t * 16 + ln, to_bf16x4(v));
       }
+    };
+    bool mid;
+    if (l == 0) {
+      product<4>(acc[0], in, ld0, b, K0 / 32);
+      product<4>(acc[1], in + 16 * ld0, ld0, b, K0 / 32);
+      pre(0);
+      mid = sigmoid_mid(z, s);
+    } else {
+      product<KS>(acc[0], in, ld, b, KS);
+      pre(0);
+      product<KS>(acc[1], in + 16 * ld, ld, b, KS);
+      mid = sigmoid_mid(z, s);
+      interleave<2 * KS>();
+    }
+    load_frags<KS>(b, wn, KS, last ? kOut / 16 : W / 16, last ? 0 : 2 * wave);
+    put(0, mid);
+    pre(1);
+    mid = sigmoid_mid(z, s);
+    put(1, mid);
     __syncthreads();
     if (TRAIN && l + slots <= nl - 2)
       for (int i = tid; i < kTile * W / 8; i += kThreads) {
@@ -379,26 +417,31 @@ __global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Poi
     }
     float bl[2];
     for (int t = 0; t < 2; t++) bl[t] = m.b[(l - 1) * W + wave * 32 + t * 16 + ln];
-    floatx4 z4[2][2];
-    if (l == nl - 1)
-      product<1>(acc, cur, ld, c, 1);
-    else
-      product<KS>(acc, cur, ld, c, KS);
-    if (l == 1)
-      product<4>(z4, sx, ld0, b, K0 / 32);
-    else
-      product<KS>(z4, rows(l - 2), ld, b, KS);
+    floatx4 acc[2][2], z4[2][2];
+    for (int i = 0; i < 2; i++) {
+      if (l == nl - 1)
+        product<1>(acc[i], cur + i * 16 * ld, ld, c, 1);
+      else
+        product<KS>(acc[i], cur + i * 16 * ld, ld, c, KS);
+      if (l == 1)
+        product<4>(z4[i], sx + i * 16 * ld0, ld0, b, K0 / 32);
+      else
+        product<KS>(z4[i], rows(l - 2) + i * 16 * ld, ld, b, KS);
+    }
     const int j = max(l - 2, 0);  // (the last round loads what it does not use)
     load_frags<KS>(c, m.wb + m.frag(j + 1), m.N(j + 1) / 32, W / 16, 2 * wave);
     load_frags<KM>(b, m.wf + m.frag(j), m.K(j) / 32, W / 16, 2 * wave);
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < 2; i++) {
+      float z[2][4], s[2][4];
+      for (int t = 0; t < 2; t++)
+        for (int r = 0; r < 4; r++) z[t][r] = z4[i][t][r] + bl[t];
+      if (!sigmoid_mid(z, s)) sigmoid_rest(z, s);
       for (int t = 0; t < 2; t++) {
-        float z[4], s[4];
-        for (int r = 0; r < 4; r++) z[r] = z4[i][t][r] + bl[t];
-        sigmoid4(z, s);
-        for (int r = 0; r < 4; r++) z[r] = acc[i][t][r] * (s[r] * (1.0f + z[r] * (1.0f - s[r])));
-        put4(nxt, ld, m.dz + m.out(l - 1), p0, W, i * 16 + lp, wave * 32 + t * 16 + ln, to_bf16x4(z));
+        float v[4];
+        for (int r = 0; r < 4; r++) v[r] = acc[i][t][r] * (s[t][r] * (1.0f + z[t][r] * (1.0f - s[t][r])));
+        put4(nxt, ld, m.dz + m.out(l - 1), p0, W, i * 16 + lp, wave * 32 + t * 16 + ln, to_bf16x4(v));
       }
+    }
     __syncthreads();
   }
 }
