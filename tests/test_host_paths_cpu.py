@@ -1,0 +1,62 @@
+"""The library's host code over a stand-in HIP runtime (fake_hip.c): what
+must hold whatever the kernels compute.  Each case is a program of its own, as
+the stand-in has to be loaded before libusg.so."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+HEAD = """
+import ctypes, sys, threading
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from tmp_amd import mesh, usg
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["gcc", "-O2", "-std=gnu11", "-shared", "-fPIC", os.path.join(HERE, "fake_hip.c"), "-o", so],
+                   check=True)
+    return so
+
+
+def run(fake, body):
+    r = subprocess.run([sys.executable, "-c", HEAD + body, fake, os.path.dirname(HERE)], capture_output=True,
+                       text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_calls_of_several_threads_on_one_context(fake):
+    """Fields of several transfer buffers read by one thread beside another
+    that reads a second field, and a third that sets the same state again:
+    every read gives its own field's values."""
+    run(fake, """
+m = mesh.rect(300, 301, bottom=mesh.WALL)
+s = usg.Solver(m, flow=usg.EULER)
+r = np.random.default_rng(1)
+U, W = r.uniform(1, 2, (s.nc, 4)), r.uniform(3, 4, (s.nc, 4))
+s.set_state(U, W)
+bad = []
+def read(fid, want):
+    for _ in range(40):
+        if not np.array_equal(s.field(fid), want):
+            bad.append(fid)
+def write():
+    for _ in range(20):
+        s.set_state(U, W)
+def small():
+    for _ in range(200):
+        if s.forces() != (0.0, 0.0):
+            bad.append("forces")
+ts = [threading.Thread(target=read, args=a) for a in ((usg.F_PRIM, U), (usg.F_CONS, W))]
+ts += [threading.Thread(target=write), threading.Thread(target=small)]
+for t in ts: t.start()
+for t in ts: t.join()
+assert not bad, bad
+""")

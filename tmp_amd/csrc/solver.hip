@@ -2091,10 +2091,13 @@ struct DevBuf {
 // buffers in turn, and the two invariant flags.  512 KB takes the bus 9 us,
 // which covers a launch; smaller fields go in one piece, without the event
 // that costs 5 us.  A buffer is free, or its last launch is behind its event
-// or somewhere on the stream.
+// or somewhere on the stream.  A call holds the lock from its first use of a
+// buffer or the flags until it has read them or the stream is done with them:
+// threads may read fields of one context side by side.
 constexpr size_t kStageLen = 512 * 1024 / sizeof(double);
 constexpr int kStageBufs = 4;
 struct Stage {
+  std::mutex lock;
   double *p = nullptr;
   int *flags = nullptr;
   hipEvent_t ev[kStageBufs] = {};
@@ -2707,6 +2710,7 @@ static int ensure_norms(usg_ctx *c, int n) {
 // the reference's message.  In a batch, failed cases are frozen by the
 // sweep kernels and reported through usg_case_status; the call succeeds.
 static int check_err(usg_ctx *c) {
+  std::lock_guard<std::mutex> lock(c->stage.lock);
   int *h = c->stage.flags;
   hipLaunchKernelGGL(k_err_host, dim3(1), dim3(64), 0, c->stream, c->ds.err, h);
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -2736,6 +2740,7 @@ static int make_stage(usg_ctx *c) {
   return USG_OK;
 }
 
+// (the functions that take, mark and drain buffers are called with the lock)
 // Waits for the stream; no buffer is in use after it.
 static int stage_drain(usg_ctx *c) {
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -2764,6 +2769,7 @@ static int stage_mark(usg_ctx *c, int b, bool event) {
 // memory and the change of layout there; 60 x 4 values in 12 us against 21.
 template <typename T>
 static int to_host(usg_ctx *c, const T *dev, int lv, int n, bool paired, double *out) {
+  std::lock_guard<std::mutex> lock(c->stage.lock);
   const size_t total = (size_t)n << lv;
   const long chunks = (long)((total + kStageLen - 1) / kStageLen);
   int bufs[kStageBufs], rc;
@@ -2791,7 +2797,7 @@ static int to_host(usg_ctx *c, const T *dev, int lv, int n, bool paired, double 
 }
 
 // A device array from host rows, by the same buffers the other way; the caller
-// drains them before it returns.
+// holds the lock and drains them before it returns.
 static int from_host(usg_ctx *c, const double *src, int lv, int n, bool paired, double *dev) {
   const size_t total = (size_t)n << lv;
   for (size_t first = 0; first < total; first += kStageLen) {
@@ -3211,6 +3217,7 @@ int usg_init_freestream(usg_ctx *c) {
 
 int usg_set_prim(usg_ctx *c, const double *U, const double *turb) {
   if (!c || !U) return fail(USG_ERR_ARG, "null argument");
+  std::lock_guard<std::mutex> lock(c->stage.lock);
   int rc = clear_case_status(c);
   if (rc) return rc;
   const int nc = c->hm.nc;
@@ -3233,6 +3240,7 @@ int usg_set_state(usg_ctx *c, const double *U, const double *W, const double *tu
   const bool sst = c->prm.flow == USG_SST;
   if (sst && (!turb || !mut)) return fail(USG_ERR_ARG, "SST state needs turb and mut");
   const int nc = c->hm.nc;
+  std::lock_guard<std::mutex> lock(c->stage.lock);
   int rc = clear_case_status(c);
   if (rc) return rc;
   if ((rc = from_host(c, U, 2, nc, true, c->ds.U))) return rc;
