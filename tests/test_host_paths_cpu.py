@@ -60,3 +60,24 @@ for t in ts: t.start()
 for t in ts: t.join()
 assert not bad, bad
 """)
+
+
+def test_refused_copy_of_the_error_flags_is_an_error(fake):
+    """A check of a residual whose flags could not be fetched is not a pass,
+    neither the first one nor one after a good one."""
+    run(fake, """
+import os
+for good in (0, 1):
+    s = usg.Solver(mesh.rect(4, 3), flow=usg.EULER)
+    for _ in range(good):
+        s.residual()
+    os.environ["FAKE_HIP_REFUSE"] = "k_err_host"
+    try:
+        s.residual()
+    except usg.UsgError as e:
+        assert "invalid argument" in str(e), e
+    else:
+        raise SystemExit("the check passed")
+    os.environ["FAKE_HIP_REFUSE"] = ""
+    s.residual()
+""")

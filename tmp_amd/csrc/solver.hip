@@ -2713,6 +2713,7 @@ static int check_err(usg_ctx *c) {
   std::lock_guard<std::mutex> lock(c->stage.lock);
   int *h = c->stage.flags;
   hipLaunchKernelGGL(k_err_host, dim3(1), dim3(64), 0, c->stream, c->ds.err, h);
+  HIPCHK(hipGetLastError());  // (a refused launch leaves the flags of an earlier call)
   HIPCHK(hipStreamSynchronize(c->stream));
   if (h[0] || h[1]) {
     HIPCHK(hipMemsetAsync(c->ds.err, 0, 2 * sizeof(int), c->stream));
