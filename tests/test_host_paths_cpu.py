@@ -81,3 +81,16 @@ for good in (0, 1):
     os.environ["FAKE_HIP_REFUSE"] = ""
     s.residual()
 """)
+
+
+def test_wide_levels_after_a_mesh_of_narrower_ones(fake):
+    """The most LDS a kernel may take belongs to the kernel, not to the mesh:
+    a solver with a ring of 98 KB still runs when one with 4 KB was made after
+    it."""
+    run(fake, """
+wide = usg.Solver(mesh.rect(512, 515, bottom=mesh.WALL), flow=usg.SST)
+narrow = usg.Solver(mesh.rect(20, 40, bottom=mesh.WALL), flow=usg.SST)
+for s in (narrow, wide, narrow):
+    s.graphs(False)  # the stand-in has none
+    s.lusgs(2)
+""")

@@ -2429,11 +2429,13 @@ static int sweep_launches(const usg_ctx *c) {
 // cells of a case: two rounds of chunks, where the launch is about as fast.
 constexpr int kLevelMin = 12, kLevelWidth = 8 * kLevelCells;
 
+// Lets k_levels take `limit` bytes of LDS, the device's most: what is set holds
+// for every context, so never a context's own need.
 template <int FLOW>
-static bool level_lds_limit(size_t bytes) {
+static bool level_lds_limit(int limit) {
   for (const void *f : {reinterpret_cast<const void *>(&k_levels<FLOW, true>),
                         reinterpret_cast<const void *>(&k_levels<FLOW, false>)})
-    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, limit) != hipSuccess) return false;
   return true;
 }
 
@@ -2553,9 +2555,9 @@ static int build_levels(usg_ctx *c) {
   const size_t lds = (size_t)kLevelRing * std::max(f.width, b.width) * sizeof(double) *
                      (c->prm.flow == USG_SST ? level_vars<USG_SST>() : level_vars<USG_EULER>());
   if (lds > (size_t)limit) return USG_OK;
-  const bool ok = c->prm.flow == USG_EULER     ? level_lds_limit<USG_EULER>(lds)
-                  : c->prm.flow == USG_LAMINAR ? level_lds_limit<USG_LAMINAR>(lds)
-                                               : level_lds_limit<USG_SST>(lds);
+  const bool ok = c->prm.flow == USG_EULER     ? level_lds_limit<USG_EULER>(limit)
+                  : c->prm.flow == USG_LAMINAR ? level_lds_limit<USG_LAMINAR>(limit)
+                                               : level_lds_limit<USG_SST>(limit);
   if (!ok) {
     (void)hipGetLastError();  // the sweeps keep their launches
     return USG_OK;
