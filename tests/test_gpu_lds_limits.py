@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from tmp_amd import mesh as MM
-from tmp_amd import usg
+from tmp_amd import mlp, usg
 
 pytestmark = pytest.mark.gpu
 
@@ -19,3 +19,18 @@ def test_wide_levels_after_a_mesh_of_narrower_ones():
             s.lusgs(2)
             U.append(s.U)
     assert np.array_equal(U[0], U[1])
+
+
+def test_deep_network_after_a_shallow_one():
+    rng = np.random.default_rng(2)
+    x, y = rng.normal(size=(70, 128)).astype(np.float32), rng.normal(size=(70, 4)).astype(np.float32)
+    got = []
+    for between in (False, True):
+        g = mlp.MLP(128, 256, 8, 4)
+        g.set_params(*[np.random.default_rng(3).normal(0, 0.1, n) for n in (g.nw, g.nb)])
+        if between:
+            mlp.MLP(20, 256, 2, 2).close()
+        got.append((g.predict(x),) + g.gradients(x, y))
+        g.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

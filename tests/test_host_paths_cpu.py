@@ -94,3 +94,16 @@ for s in (narrow, wide, narrow):
     s.graphs(False)  # the stand-in has none
     s.lusgs(2)
 """)
+
+
+def test_deep_network_after_a_shallow_one(fake):
+    """As above for the networks of one width: rows of all layers in LDS."""
+    run(fake, """
+from tmp_amd import mlp
+def use(g):
+    g.gradients(np.zeros((5, g.nin)), np.zeros((5, g.nout)))
+    g.predict(np.zeros((5, g.nin)))
+deep, shallow = mlp.MLP(128, 256, 8, 4), mlp.MLP(20, 256, 2, 2)
+for g in (shallow, deep, shallow):
+    use(g)
+""")

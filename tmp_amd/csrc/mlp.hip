@@ -729,10 +729,9 @@ int net_lds(usg_mlp *m, int limit) {
   m->slots = std::max(m->slots, 2);
   m->lds_train = x + y + (2 + m->slots) * row;
   m->lds_predict = x + 2 * row;
-  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_net<W, true>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)m->lds_train));
-  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_net<W, false>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)m->lds_predict));
+  // what is set holds for every network of this width: the device's most
+  for (const void *f : {reinterpret_cast<const void *>(&k_net<W, true>), reinterpret_cast<const void *>(&k_net<W, false>)})
+    HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, limit));
   return 0;
 }
 
