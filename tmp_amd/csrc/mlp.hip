@@ -127,10 +127,12 @@ __device__ __forceinline__ float exp_mid(float x) {
   const float n = __builtin_rintf(t);
   return __builtin_ldexpf(__builtin_amdgcn_exp2f((t - n) + lo), (int)n);
 }
-// 1 / x, correctly rounded for 1 <= x < 2^126: two Newton steps on the
-// approximate reciprocal, the second on the quotient's remainder (equal to the
-// quotient for every such x).  No operand needs the scaling of a general
-// division.
+// 1 / x for 1 <= x < 2^126: two Newton steps on the approximate reciprocal, the
+// second on the quotient's remainder.  From a start within one unit they give
+// the rounded quotient, but for a mantissa of all ones, where the start has to
+// be it already, or the result is one unit below.  With gfx950's v_rcp_f32 no
+// x of the range differs from the quotient (all compared).  No operand needs
+// the scaling of a general division.
 __device__ __forceinline__ float recip_mid(float x) {
   float r = __builtin_amdgcn_rcpf(x);
   r = __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
