@@ -2,8 +2,10 @@
  * where there is no GPU: device memory is host memory, every call is done
  * when it returns, a wait takes 0.2 ms, and no kernel does anything but the
  * copies to and from pinned memory.  A launch is refused as HIP refuses it:
- * dynamic LDS above the function's maximum (64 KB until it is set), or a name
- * that contains $FAKE_HIP_REFUSE.  Loaded with RTLD_GLOBAL before libusg.so. */
+ * dynamic LDS above the function's maximum (64 KB until it is set), more than
+ * 65536 blocks along y or z, or a name that contains $FAKE_HIP_REFUSE.  Copies
+ * and fills of more than 256 MB are not made.  Loaded with RTLD_GLOBAL before
+ * libusg.so. */
 #include <stddef.h>
 #include <stdlib.h>
 #include <string.h>
@@ -75,8 +77,8 @@ static void copy_fields(const char *name, void **a) {
 int hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **a, size_t lds, void *stream) {
   const int i = find(f);
   const char *refuse = getenv("FAKE_HIP_REFUSE");
-  (void)grid, (void)block, (void)stream;
-  if (i < 0 || lds > fn[i].lds || (refuse && *refuse && strstr(fn[i].name, refuse))) return last = kInvalid;
+  (void)block, (void)stream;
+  if (i < 0 || lds > fn[i].lds || grid.y > 65536 || grid.z > 65536 || (refuse && *refuse && strstr(fn[i].name, refuse))) return last = kInvalid;
   if (strstr(fn[i].name, "k_to_host") || strstr(fn[i].name, "k_from_host")) copy_fields(fn[i].name, a);
   if (strstr(fn[i].name, "k_err_host")) memcpy(*(void **)a[1], *(void **)a[0], 2 * sizeof(int));
   return kOk;
@@ -114,7 +116,7 @@ int hipHostMalloc(void **p, size_t n, unsigned flags) {
 int hipHostFree(void *p) { return free(p), kOk; }
 int hipMemcpy(void *d, const void *s, size_t n, int kind) {
   (void)kind;
-  if (n) memcpy(d, s, n);
+  if (n && n <= 1u << 28) memcpy(d, s, n);
   return kOk;
 }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *stream) {
@@ -123,7 +125,8 @@ int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *stream) {
 }
 int hipMemsetAsync(void *d, int v, size_t n, void *stream) {
   (void)stream;
-  return memset(d, v, n), kOk;
+  if (n <= 1u << 28) memset(d, v, n);
+  return kOk;
 }
 
 int hipStreamCreate(void **s) { return *s = malloc(1), kOk; }

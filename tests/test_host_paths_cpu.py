@@ -107,3 +107,12 @@ deep, shallow = mlp.MLP(128, 256, 8, 4), mlp.MLP(20, 256, 2, 2)
 for g in (shallow, deep, shallow):
     use(g)
 """)
+
+
+def test_more_layers_than_a_grid_has_rows(fake):
+    """A network of more than 65536 layers: its weights are packed layer by
+    layer, and a launch has at most 65536 blocks along y."""
+    run(fake, """
+from tmp_amd import mlp
+mlp.MLP(1, 64, 65540, 1).close()
+""")

@@ -635,15 +635,18 @@ __global__ void k_mfma_check(const bf16 *a, const bf16 *b, float *d) {
   for (int r = 0; r < 4; r++) d[((lane / 16) * 4 + r) * 16 + lane % 16] = c[r];
 }
 
-// BF16 fragments of a layer's weights (blockIdx.y) from the FP32 masters; the
-// padding stays zero.
+// BF16 fragments of the layers' weights (blockIdx.y, and every kPackRows layers
+// on) from the FP32 masters; the padding stays zero.
+constexpr int kPackRows = 32768;  // (a launch has at most 65536 blocks along y)
 __global__ __launch_bounds__(256) void k_pack(const Net m) {
-  const int l = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= m.k(l) * m.n(l)) return;
-  const int k = i / m.n(l), n = i % m.n(l);
-  const bf16 h = to_bf16(m.w[m.ow(l) + i]);
-  m.wf[m.frag(l) + wf_index(k, n, m.N(l))] = h;
-  m.wb[m.frag(l) + wb_index(k, n, m.K(l))] = h;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  for (int l = blockIdx.y; l < m.nl; l += kPackRows) {
+    if (i >= m.k(l) * m.n(l)) continue;
+    const int k = i / m.n(l), n = i % m.n(l);
+    const bf16 h = to_bf16(m.w[m.ow(l) + i]);
+    m.wf[m.frag(l) + wf_index(k, n, m.N(l))] = h;
+    m.wb[m.frag(l) + wb_index(k, n, m.K(l))] = h;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -861,7 +864,7 @@ int usg_mlp_set_params(usg_mlp *m, const float *w, const float *b) {
   for (float *p : {m->mo.m1, m->mo.m2}) HIPCHK(hipMemsetAsync(p, 0, m->nw * sizeof(float), m->s));
   for (float *p : {m->mo.m1b, m->mo.m2b}) HIPCHK(hipMemsetAsync(p, 0, m->nb * sizeof(float), m->s));
   const int most = std::max(m->d.nin, m->d.width) * m->d.width;
-  hipLaunchKernelGGL(k_pack, dim3((most + 255) / 256, m->net.nl), dim3(256), 0, m->s, m->net);
+  hipLaunchKernelGGL(k_pack, dim3((most + 255) / 256, std::min(m->net.nl, kPackRows)), dim3(256), 0, m->s, m->net);
   HIPCHK(hipGetLastError());
   m->step = 0;
   HIPCHK(hipStreamSynchronize(m->s));
