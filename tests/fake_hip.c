@@ -4,9 +4,11 @@
  * copies to and from pinned memory.  A launch is refused as HIP refuses it:
  * dynamic LDS above the function's maximum (64 KB until it is set), more than
  * 65536 blocks along y or z, or a name that contains $FAKE_HIP_REFUSE.  Copies
- * and fills of more than 256 MB are not made.  Loaded with RTLD_GLOBAL before
+ * and fills of more than 256 MB are not made.  Of k_levels the order of work and
+ * barriers is gone through on the tables it is given.  Loaded with RTLD_GLOBAL before
  * libusg.so. */
 #include <stddef.h>
+#include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 #include <unistd.h>
@@ -74,12 +76,47 @@ static void copy_fields(const char *name, void **a) {
       (*(double **)a[1])[e] = single ? (*(float **)a[0])[p] : (*(double **)a[0])[p];
   }
 }
+/* k_levels: its groups take the chunks of a case in turn and meet at barriers.
+ * Every group has to execute as many as there are levels, and to be past the
+ * barrier of a chunk's level, and not past the next one, when it works on it. */
+enum { kGroups = 4 };
+typedef struct {
+  int n;
+  const int *pos, *cell, *code, (*chunk)[4], *coff;
+  void *rec, *base, *diag, *tbase, *tdiag, *off;
+} levels;
+static void check(int ok, const char *what) {
+  if (ok) return;
+  fprintf(stderr, "k_levels: %s\n", what);
+  exit(3);
+}
+static void check_levels(const levels *w, int ncase) {
+  for (int c = 0; c < ncase; c++) {
+    const int n0 = w->coff[c], n1 = w->coff[c + 1];
+    int begun = 0;
+    check((n1 - n0) % kGroups == 0, "a case's chunks are no whole rounds");
+    for (int i = n0; i < n1; i++) begun += w->chunk[i][3] & 1;
+    for (int g = 0; g < kGroups && n0 < n1; g++) {
+      int waits = 0;
+      for (int i = 0; i < g; i++) waits += w->chunk[n0][3] >> i & 1;
+      for (int n = n0 + g; n < n1; n += kGroups) {
+        int level = 0;
+        for (int i = n0; i <= n; i++) level += w->chunk[i][3] & 1;
+        waits += w->chunk[n][3] & 1;
+        check(waits == level, "a group works on a chunk of another level");
+        for (int i = 1; i < kGroups; i++) waits += w->chunk[n][3] >> i & 1;
+      }
+      check(waits == begun, "groups meet different numbers of barriers");
+    }
+  }
+}
 int hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **a, size_t lds, void *stream) {
   const int i = find(f);
   const char *refuse = getenv("FAKE_HIP_REFUSE");
   (void)block, (void)stream;
   if (i < 0 || lds > fn[i].lds || grid.y > 65536 || grid.z > 65536 || (refuse && *refuse && strstr(fn[i].name, refuse))) return last = kInvalid;
   if (strstr(fn[i].name, "k_to_host") || strstr(fn[i].name, "k_from_host")) copy_fields(fn[i].name, a);
+  if (strstr(fn[i].name, "k_levels")) check_levels((const levels *)a[1] + !strstr(fn[i].name, "ELb1E"), grid.x);
   if (strstr(fn[i].name, "k_err_host")) memcpy(*(void **)a[1], *(void **)a[0], 2 * sizeof(int));
   return kOk;
 }

@@ -116,3 +116,18 @@ def test_more_layers_than_a_grid_has_rows(fake):
 from tmp_amd import mlp
 mlp.MLP(1, 64, 65540, 1).close()
 """)
+
+
+def test_groups_of_the_level_sweeps_meet_the_same_barriers(fake):
+    """For levels of one cell to the widest, chunks and rounds around their
+    sizes, and batches with cases of no narrow level."""
+    run(fake, """
+ms = [mesh.rect(a, b, jitter=0.1, seed=1, bottom=mesh.WALL)
+      for a, b in ((2, 30), (9, 40), (63, 70), (64, 70), (65, 70), (129, 150), (256, 260), (257, 260), (512, 515))]
+ms.append(mesh.airfoil_hybrid(ni=64, dy1=1e-3, rfar=10.0))
+one = [usg.Solver(m, flow=usg.EULER) for m in ms]
+assert all(sum(s.waves()) > 14 for s in one)
+for s in one + [usg.BatchSolver([mesh.rect(1, 1)] + ms[i:] + [mesh.rect(2, 2)], flow=usg.EULER) for i in (0, 3, 7)]:
+    s.graphs(False)  # the stand-in has none
+    s.lusgs(1)
+""")

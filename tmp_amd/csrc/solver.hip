@@ -1522,6 +1522,22 @@ __device__ __forceinline__ double quad_lane(double x) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// The barrier of k_levels, whose groups come to it at different places of the
+// code.  HIP's rule for __syncthreads wants every thread at one place; this is
+// the instruction itself, which counts waves wherever they are, with the same
+// fences.  Each group executes it once for every chunk that begins a level:
+// before its first chunk those of the groups ahead of it (`before`), then, with
+// each chunk of its own, those of that chunk and the G - 1 after it
+// (LevelSweep::chunk); a case's chunks are whole rounds, so the groups' counts
+// are equal.  (One place in a loop that all groups go through together makes
+// the compiler wait for the records in every turn: 200 levels of 25 cells 325
+// -> 570 us an iteration.)
+__device__ __forceinline__ void level_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // Bound by the latency of one level: barrier, LDS read, flux, four-lane sum,
 // quotient, LDS write.  Everything else is taken out of that chain: the groups
 // take the chunks in turn, and a group between two chunks of its own loads
@@ -1674,17 +1690,17 @@ __global__ __launch_bounds__(kLevelThreads) void k_levels(const DevState s, cons
   ch2 = place(n + 2 * G);
   const int before = place(n0).w;  // the levels that begin with the other groups' first chunks
   for (int i = 0; i < group; i++)
-    if (before >> i & 1) __syncthreads();
+    if (before >> i & 1) level_barrier();
   for (; n < n1; n += G) {
     const int begins = ch.w;
     flux();
-    if (begins & 1) __syncthreads();
+    if (begins & 1) level_barrier();
     work();
-    if (begins & 2) __syncthreads();
+    if (begins & 2) level_barrier();
     next(n);
 #pragma unroll
     for (int i = 2; i < G; i++)
-      if (begins >> i & 1) __syncthreads();
+      if (begins >> i & 1) level_barrier();
   }
 }
 
