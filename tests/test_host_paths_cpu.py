@@ -123,7 +123,7 @@ def test_groups_of_the_level_sweeps_meet_the_same_barriers(fake):
     sizes, and batches with cases of no narrow level."""
     run(fake, """
 ms = [mesh.rect(a, b, jitter=0.1, seed=1, bottom=mesh.WALL)
-      for a, b in ((2, 30), (9, 40), (63, 70), (64, 70), (65, 70), (129, 150), (256, 260), (257, 260), (512, 515))]
+      for a, b in ((2, 30), (9, 40), (63, 70), (64, 70), (65, 70), (129, 150), (256, 260), (257, 260), (512, 515), (513, 515))]
 ms.append(mesh.airfoil_hybrid(ni=64, dy1=1e-3, rfar=10.0))
 one = [usg.Solver(m, flow=usg.EULER) for m in ms]
 assert all(sum(s.waves()) > 14 for s in one)
