@@ -88,6 +88,8 @@ struct Net {
   __host__ __device__ long out(int l) const { return l * P * W; }
   __host__ __device__ long ow(int l) const { return l == 0 ? 0 : (long)nin * W + (long)(l - 1) * W * W; }
   __host__ __device__ long ob(int l) const { return (long)l * W; }
+  __host__ __device__ long weights() const { return ow(nl - 1) + (long)W * nout; }
+  __host__ __device__ long params() const { return weights() + ob(nl - 1) + nout; }
 };
 __host__ __device__ __forceinline__ size_t wf_index(int k, int n, int N) {
   return ((size_t)((k / 32) * (N / 16) + n / 16) * 64 + (k % 32) / 8 * 16 + n % 16) * 8 + k % 8;
@@ -465,6 +467,13 @@ __global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Poi
 // us, against 192 us for a launch per layer for the partial products, the bias
 // sums and each update, with the partial products in memory.
 // ---------------------------------------------------------------------------
+// A network of few such blocks leaves CUs idle, and its one walk over the points
+// of a large batch is the time: the points are then split over `splits` rows of
+// blocks (each a whole number of kSplit steps), which leave partial gradients
+// in memory, and k_apply adds these up in order and takes Adam's step
+// (weight_splits).  A training step, one walk -> split: 64 x 2 layers, 16 384
+// points 99 -> 64 us, 131 072 points 474 -> 179 us; 128 x 2, 400 000 points 1890
+// -> 653 us; 256 x 3, 32 768 points 223 -> 183 us.
 struct WeightTile {
   int layer, k0, n0;  // layer -1: no work; k0 -1: the bias sums of 16 columns
 };
@@ -475,6 +484,8 @@ struct Moments {
   float *m1, *m2, *m1b, *m2b;
 };
 constexpr int kFlight = 16;
+constexpr int kSplit = 64;  // steps (of 32 points): 8 chunks, an iteration of bias_sums
+constexpr int kSplitSteps = 512;
 
 // One Adam step on parameter p[o].
 __device__ __forceinline__ float adam(float *p, float *m1, float *m2, size_t o, float g, const AdamStep &st) {
@@ -490,14 +501,15 @@ __device__ __forceinline__ float adam(float *p, float *m1, float *m2, size_t o, 
 // Bias gradients of columns n0 .. n0 + 15 of layer l (two waves): a lane takes
 // one column of one chunk, sums the 8-point blocks j, j + 8, ... of the chunk
 // for each j, then the eight sums, and the chunks add up in order.
+// (steps first .. end - 1 of 32 points, four 8-point blocks each)
 template <bool ADAM>
-__device__ __forceinline__ void bias_sums(const Net &m, int l, int n0, const AdamStep &st, const Moments &mo,
-                                          float *gb) {
+__device__ __forceinline__ void bias_sums(const Net &m, int l, int n0, int first, int end, const AdamStep &st,
+                                          const Moments &mo, float *gb) {
   __shared__ float part[8][16];
-  const int tid = threadIdx.x, N = m.N(l), c0 = tid / 16, nblk = (int)(m.P / 8);
+  const int tid = threadIdx.x, N = m.N(l), c0 = tid / 16, nblk = end * 4;
   const bf16 *d = m.dz + m.out(l);
   float sum = 0.0f;
-  for (int b0 = 0; b0 < nblk; b0 += 8 * (kChunk / 8)) {
+  for (int b0 = first * 4; b0 < nblk; b0 += 8 * (kChunk / 8)) {
     const int b = b0 + c0 * (kChunk / 8);
     float s[8];
 #pragma unroll
@@ -534,20 +546,29 @@ template <bool ADAM>
 __global__ __launch_bounds__(128, 1) void k_weights(const Net m, const WeightTile *__restrict__ tiles,
                                                     const AdamStep st, const Moments mo, float *__restrict__ gw,
                                                     float *__restrict__ gb) {
-  const WeightTile tl = tiles[blockIdx.x];
+  // row r of blocks: the tiles of a layer one XCD further on than row r - 1's
+  const int row = blockIdx.y, rows = gridDim.y;
+  const WeightTile tl = tiles[blockIdx.x / 8 * 8 + (blockIdx.x + 8 - row % 8) % 8];
+  const int units = (int)((m.P / 32 + kSplit - 1) / kSplit);
+  const int first = units * row / rows * kSplit, end = min(units * (row + 1) / rows * kSplit, (int)(m.P / 32));
+  if (rows > 1) {
+    gw += (size_t)row * m.params();
+    gb += (size_t)row * m.params();
+  }
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int l = tl.layer, n0 = tl.n0 + wave * 32;
   if (l < 0) return;
   if (tl.k0 < 0) {
-    bias_sums<ADAM>(m, l, tl.n0, st, mo, gb);
+    bias_sums<ADAM>(m, l, tl.n0, first, end, st, mo, gb);
     return;
   }
   const int K = m.K(l), N = m.N(l), rk = m.k(l), rn = m.n(l);
   if (n0 >= N) return;
-  const int nstep = (int)(m.P / 32);  // a multiple of 4
+  const int nstep = end - first;  // a multiple of 4
   // the step to load next (its last one again past the end): uniform bases
   // and a lane's offset, so that a step costs a few scalar additions
-  const bf16 *x = m.in + m.inp(l) + tl.k0 / 16 * 512, *d = m.dz + m.out(l) + n0 / 16 * 512;
+  const bf16 *x = m.in + m.inp(l) + (size_t)first * 32 * K + tl.k0 / 16 * 512,
+             *d = m.dz + m.out(l) + (size_t)first * 32 * N + n0 / 16 * 512;
   int left = nstep - 1;
   bf16x8 a[kFlight][2], b[kFlight][2];
   auto fetch = [&](int slot) {
@@ -602,6 +623,31 @@ __global__ __launch_bounds__(128, 1) void k_weights(const Net m, const WeightTil
         m.wf[m.frag(l) + wf_index(k, n, N)] = h;
         m.wb[m.frag(l) + wb_index(k, n, K)] = h;
       }
+}
+
+// The gradients of layer blockIdx.y: the sums over the splits' partial ones, in
+// order, and Adam's step on them (or the gradients themselves).
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_apply(const Net m, int splits, const float *__restrict__ part,
+                                               const AdamStep st, const Moments mo, float *__restrict__ gw,
+                                               float *__restrict__ gb) {
+  const int l = blockIdx.y, rk = m.k(l), rn = m.n(l), nw = rk * rn;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= nw + rn) return;
+  const size_t o = i < nw ? m.ow(l) + i : m.ob(l) + (i - nw);
+  const float *p = part + (i < nw ? o : m.weights() + o);
+  float g = p[0];
+  for (int q = 1; q < splits; q++) g += p[(size_t)q * m.params()];
+  if (!ADAM) {
+    (i < nw ? gw : gb)[o] = g;
+  } else if (i >= nw) {
+    adam(m.b, mo.m1b, mo.m2b, o, g, st);
+  } else {
+    const int k = i / rn, n = i % rn;
+    const bf16 h = to_bf16(adam(m.w, mo.m1, mo.m2, o, g, st));
+    m.wf[m.frag(l) + wf_index(k, n, m.N(l))] = h;
+    m.wb[m.frag(l) + wb_index(k, n, m.K(l))] = h;
+  }
 }
 
 // Batch losses of an epoch, one block per step: scale * (sum of the step's n
@@ -671,13 +717,14 @@ struct usg_mlp {
   std::vector<void *> allocs;
   long step = 0;
   WeightTile *d_tiles = nullptr;
-  int ntiles = 0;
+  int ntiles = 0, nwork = 0;  // blocks of k_weights, and those of them with work
+  int cus = 0;
   int slots = 0;              // layers whose rows LDS holds in training
   size_t lds_train = 0, lds_predict = 0;
   // training buffers for `cap` points (Net's in, dz and h)
   int cap = 0;
   std::vector<void *> bufs;
-  Buf x, y, g, lossp, losses, idx;
+  Buf x, y, g, part, lossp, losses, idx;
   // resident training set
   bf16 *xs = nullptr;
   float *ys = nullptr;
@@ -768,13 +815,49 @@ int build_tiles(usg_mlp *m) {
   for (int l = 0; l < m->net.nl; l++)
     for (int n0 = 0; n0 < m->net.n(l); n0 += 16) by[l % 8].push_back({l, -1, n0});
   size_t most = 0;
-  for (auto &v : by) most = std::max(most, v.size());
+  for (auto &v : by) {
+    most = std::max(most, v.size());
+    m->nwork += (int)v.size();
+  }
   for (size_t i = 0; i < most; i++)
     for (auto &v : by) all.push_back(i < v.size() ? v[i] : WeightTile{-1, 0, 0});
   m->ntiles = (int)all.size();
   if (int rc = dalloc(m->allocs, &m->d_tiles, all.size())) return rc;
   HIPCHK(hipMemcpy(m->d_tiles, all.data(), all.size() * sizeof(WeightTile), hipMemcpyHostToDevice));
   return 0;
+}
+
+// Rows of blocks that k_weights splits a batch's points over: as many as the
+// CUs take beside one another, if the second launch is repaid.  Split from 64
+// steps on, training gained at every size (8192 points: 84 -> 69 us), but the
+// gradients of one batch lost (4096 points: 109 -> 130 us, 8192: 147 -> 159,
+// 16 384: 227 -> 224).
+int weight_splits(const usg_mlp *m) {
+  const int steps = (int)(m->net.P / 32), units = (steps + kSplit - 1) / kSplit;
+  return steps < kSplitSteps ? 1 : std::max(1, std::min(units, m->cus / m->nwork));
+}
+
+// The partial gradients' memory, before a step's first launch.
+int ensure_parts(usg_mlp *m) {
+  const int splits = weight_splits(m);
+  return splits > 1 ? grow(m, m->part, (size_t)splits * m->net.params() * sizeof(float)) : 0;
+}
+
+// Weight and bias gradients of the points k_net went through, and Adam on them
+// (or the gradients themselves, into gw and gb).
+template <bool ADAM>
+void weights(usg_mlp *m, const AdamStep &st, float *gw, float *gb) {
+  const int splits = weight_splits(m);
+  if (splits == 1) {
+    hipLaunchKernelGGL((k_weights<ADAM>), dim3(m->ntiles), dim3(128), 0, m->s, m->net, m->d_tiles, st, m->mo, gw, gb);
+    return;
+  }
+  float *part = (float *)m->part.p;
+  hipLaunchKernelGGL((k_weights<false>), dim3(m->ntiles, splits), dim3(128), 0, m->s, m->net, m->d_tiles, st, m->mo,
+                     part, part + m->nw);
+  const int most = (std::max(m->d.nin, m->d.width) + 1) * m->d.width;
+  hipLaunchKernelGGL((k_apply<ADAM>), dim3((most + 255) / 256, m->net.nl), dim3(256), 0, m->s, m->net, splits, part, st,
+                     m->mo, gw, gb);
 }
 
 }  // namespace usgmlp
@@ -798,7 +881,7 @@ int usg_mlp_destroy(usg_mlp *m) {
   if (m->s) hipStreamSynchronize(m->s);
   for (void *p : m->bufs) hipFree(p);
   for (void *p : m->allocs) hipFree(p);
-  for (Buf *b : {&m->x, &m->y, &m->g, &m->lossp, &m->losses, &m->idx})
+  for (Buf *b : {&m->x, &m->y, &m->g, &m->part, &m->lossp, &m->losses, &m->idx})
     if (b->p) hipFree(b->p);
   if (m->xs) hipFree(m->xs);
   if (m->ys) hipFree(m->ys);
@@ -827,6 +910,7 @@ static int create(usg_mlp *m) {
   for (bf16 *p : {t.wf, t.wb}) HIPCHK(hipMemsetAsync(p, 0, frags * sizeof(bf16), m->s));
   HIPCHK(hipGetDevice(&dev));
   HIPCHK(hipDeviceGetAttribute(&limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  HIPCHK(hipDeviceGetAttribute(&m->cus, hipDeviceAttributeMultiprocessorCount, dev));
   switch (d.width) {
     case 64: return net_lds<64>(m, limit);
     case 128: return net_lds<128>(m, limit);
@@ -910,14 +994,14 @@ int usg_mlp_gradients(usg_mlp *m, const float *x, const float *y, int n, float *
   if (!m || !x || !y || n <= 0) return fail(-1, "bad argument");
   const int P = round_up(n, 128), nbl = P / 8;
   int rc = ensure_cap(m, P);
-  if (rc || (rc = grow(m, m->lossp, nbl * sizeof(float))) || (rc = grow(m, m->g, (m->nw + m->nb) * sizeof(float))))
+  if (rc || (rc = ensure_parts(m)) || (rc = grow(m, m->lossp, nbl * sizeof(float))) ||
+      (rc = grow(m, m->g, (m->nw + m->nb) * sizeof(float))))
     return rc;
   Points pt;
   if ((rc = upload_points(m, x, y, n, pt))) return rc;
   float *gw = (float *)m->g.p, *gb = gw + m->nw;
   net(m, true, P / kTile, pt, nullptr, (float *)m->lossp.p);
-  hipLaunchKernelGGL((k_weights<false>), dim3(m->ntiles), dim3(128), 0, m->s, m->net, m->d_tiles, AdamStep{},
-                     Moments{}, gw, gb);
+  weights<false>(m, AdamStep{}, gw, gb);
   HIPCHK(hipGetLastError());
   std::vector<float> lp(loss ? nbl : 0);
   if (loss) HIPCHK(hipMemcpyAsync(lp.data(), m->lossp.p, nbl * sizeof(float), hipMemcpyDeviceToHost, m->s));
@@ -964,8 +1048,8 @@ int usg_mlp_train_epoch(usg_mlp *m, const int *perm, long n, int batch, float lr
   const int P = round_up(batch, 128), nbl = P / 8;
   const long nsteps = (n + batch - 1) / batch;
   int rc = ensure_cap(m, P);
-  if (rc || (rc = grow(m, m->idx, n * sizeof(int))) || (rc = grow(m, m->lossp, (size_t)nsteps * nbl * sizeof(float))) ||
-      (rc = grow(m, m->losses, nsteps * sizeof(float))))
+  if (rc || (rc = ensure_parts(m)) || (rc = grow(m, m->idx, n * sizeof(int))) ||
+      (rc = grow(m, m->lossp, (size_t)nsteps * nbl * sizeof(float))) || (rc = grow(m, m->losses, nsteps * sizeof(float))))
     return rc;
   HIPCHK(hipMemcpyAsync(m->idx.p, perm, n * sizeof(int), hipMemcpyHostToDevice, m->s));
   float *lossp = (float *)m->lossp.p;
@@ -976,8 +1060,7 @@ int usg_mlp_train_epoch(usg_mlp *m, const int *perm, long n, int batch, float lr
         lossp + q * nbl);
     m->step++;
     const AdamStep st{lr, 1.0f - std::pow(0.9f, (float)m->step), 1.0f - std::pow(0.999f, (float)m->step)};
-    hipLaunchKernelGGL((k_weights<true>), dim3(m->ntiles), dim3(128), 0, m->s, m->net, m->d_tiles, st, m->mo, nullptr,
-                       nullptr);
+    weights<true>(m, st, nullptr, nullptr);
   }
   hipLaunchKernelGGL(k_losses, dim3((unsigned)nsteps), dim3(256), 0, m->s, lossp, nbl,
                      (float)(1.0 / ((double)batch * m->d.nout)), (float)(1.0 / ((double)nv * m->d.nout)),
