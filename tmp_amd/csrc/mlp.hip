@@ -681,18 +681,16 @@ __global__ void k_mfma_check(const bf16 *a, const bf16 *b, float *d) {
   for (int r = 0; r < 4; r++) d[((lane / 16) * 4 + r) * 16 + lane % 16] = c[r];
 }
 
-// BF16 fragments of the layers' weights (blockIdx.y, and every kPackRows layers
-// on) from the FP32 masters; the padding stays zero.
-constexpr int kPackRows = 32768;  // (a launch has at most 65536 blocks along y)
-__global__ __launch_bounds__(256) void k_pack(const Net m) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  for (int l = blockIdx.y; l < m.nl; l += kPackRows) {
-    if (i >= m.k(l) * m.n(l)) continue;
-    const int k = i / m.n(l), n = i % m.n(l);
-    const bf16 h = to_bf16(m.w[m.ow(l) + i]);
-    m.wf[m.frag(l) + wf_index(k, n, m.N(l))] = h;
-    m.wb[m.frag(l) + wb_index(k, n, m.K(l))] = h;
-  }
+// BF16 fragments of the weights of layers l0 + blockIdx.y from the FP32 masters;
+// the padding stays zero.
+constexpr int kPackLayers = 32768;  // (a launch has at most 65536 blocks along y)
+__global__ __launch_bounds__(256) void k_pack(const Net m, int l0) {
+  const int l = l0 + blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= m.k(l) * m.n(l)) return;
+  const int k = i / m.n(l), n = i % m.n(l);
+  const bf16 h = to_bf16(m.w[m.ow(l) + i]);
+  m.wf[m.frag(l) + wf_index(k, n, m.N(l))] = h;
+  m.wb[m.frag(l) + wb_index(k, n, m.K(l))] = h;
 }
 
 // ---------------------------------------------------------------------------
@@ -948,7 +946,9 @@ int usg_mlp_set_params(usg_mlp *m, const float *w, const float *b) {
   for (float *p : {m->mo.m1, m->mo.m2}) HIPCHK(hipMemsetAsync(p, 0, m->nw * sizeof(float), m->s));
   for (float *p : {m->mo.m1b, m->mo.m2b}) HIPCHK(hipMemsetAsync(p, 0, m->nb * sizeof(float), m->s));
   const int most = std::max(m->d.nin, m->d.width) * m->d.width;
-  hipLaunchKernelGGL(k_pack, dim3((most + 255) / 256, std::min(m->net.nl, kPackRows)), dim3(256), 0, m->s, m->net);
+  for (int l0 = 0; l0 < m->net.nl; l0 += kPackLayers)
+    hipLaunchKernelGGL(k_pack, dim3((most + 255) / 256, std::min(m->net.nl - l0, kPackLayers)), dim3(256), 0, m->s,
+                       m->net, l0);
   HIPCHK(hipGetLastError());
   m->step = 0;
   HIPCHK(hipStreamSynchronize(m->s));
