@@ -13,7 +13,8 @@
 // lane).  Every operand load is one 16-byte load.
 //
 // A training step is two launches: k_net (batch assembly, forward pass, loss,
-// data gradients) and k_weights (weight and bias gradients, Adam).
+// data gradients) and k_weights (weight and bias gradients, Adam); for a small
+// network on a large batch k_apply (Adam) is a third.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -227,12 +228,12 @@ __device__ __forceinline__ void put4(bf16 *rows, int ld, bf16 *op, int p0, int N
 // costs a third more matrix work but no 4-byte value per activation to memory
 // and back.  A layer's weights come from L2 into registers while the previous
 // layer's activation is in work.
-// Bound by the SiLU and its derivative: a layer's forward activation takes
-// about 4500 of its 5750 cycles, the derivative 6600 of 8900; products and
-// barriers the rest, and the first loads of the points 12000 of a block's
-// 120000 cycles.  Measured at 8 x 256 on 16384 points: 112 us, against 350 us
-// for a launch per product (and one each for the batch, the loss and the last
-// layer).  Inference of 12576 points takes 36 us, against 98 us, with the two
+// Bound by the vector instructions of the SiLU and its derivative: they issue
+// in 42 % of the SIMDs' cycles in training, whose two waves per SIMD wait for
+// data or a barrier a third of their time, and in 67 % in inference; matrix
+// instructions take 14 and 18 %.  Measured at 8 x 256 on 16384 points: 116 us,
+// against 350 us for a launch per product (and one each for the batch, the loss
+// and the last layer).  Inference of 12576 points takes 36 us, against 98 us, with the two
 // halves of a block's points one behind the other (125 VGPRs: two blocks to a
 // CU; both at once took 179 VGPRs and 45 us).
 // ---------------------------------------------------------------------------
@@ -458,15 +459,15 @@ __global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Poi
 // MFMA order), added in chunk order, so the result does not depend on the
 // launch.  Operands go straight from memory to registers, kFlight steps of 32
 // points ahead.  The bias sums are blocks of their own (beside a block's
-// products they took as long again).  Blocks of one layer share an XCD (block b: XCD b % 8, layer b % 8 of each eight), so its
-// L2 reads each operand once.  Adam runs on the sum while it is in registers:
-// FP32 master weights, then the BF16 fragments of the next step's products.
+// products they took as long again).  Blocks of one layer share an XCD (block
+// b: XCD b % 8, layer b % 8 of each eight), so its L2 reads each operand once.
+// Adam runs on the sum while it is in registers: FP32 master weights, then the
+// BF16 fragments of the next step's products.
 // Bound by the operands' way from L2 into the CUs, 8 KB per block and 32
 // points (with every block on the same 16 steps it takes 5 us less; 8 to 24
 // steps in flight make no difference).  Measured at 8 x 256, 16384 points: 60
 // us, against 192 us for a launch per layer for the partial products, the bias
 // sums and each update, with the partial products in memory.
-// ---------------------------------------------------------------------------
 // A network of few such blocks leaves CUs idle, and its one walk over the points
 // of a large batch is the time: the points are then split over `splits` rows of
 // blocks (each a whole number of kSplit steps), which leave partial gradients
@@ -474,6 +475,7 @@ __global__ __launch_bounds__(2 * W) void k_net(const Net m, int slots, const Poi
 // (weight_splits).  A training step, one walk -> split: 64 x 2 layers, 16 384
 // points 99 -> 64 us, 131 072 points 474 -> 179 us; 128 x 2, 400 000 points 1890
 // -> 653 us; 256 x 3, 32 768 points 223 -> 183 us.
+// ---------------------------------------------------------------------------
 struct WeightTile {
   int layer, k0, n0;  // layer -1: no work; k0 -1: the bias sums of 16 columns
 };
@@ -780,7 +782,8 @@ int net_lds(usg_mlp *m, int limit) {
   m->lds_train = x + y + (2 + m->slots) * row;
   m->lds_predict = x + 2 * row;
   // what is set holds for every network of this width: the device's most
-  for (const void *f : {reinterpret_cast<const void *>(&k_net<W, true>), reinterpret_cast<const void *>(&k_net<W, false>)})
+  for (const void *f :
+       {reinterpret_cast<const void *>(&k_net<W, true>), reinterpret_cast<const void *>(&k_net<W, false>)})
     HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, limit));
   return 0;
 }

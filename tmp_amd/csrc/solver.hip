@@ -158,7 +158,7 @@ __global__ __launch_bounds__(kBlock) void k_grad(const DevMesh m, const DevState
   // for.  The gathers in flight take registers (SST 113 -> 151 VGPRs, 4 -> 3
   // waves per SIMD), which the fewer waits repay.  Measured: Euler 20 k cells
   // 8.8 -> 7.3 us, 106 k 14.1 -> 12.7 us; laminar 100 k (batch) 14.9 -> 13.1
-  // us; SST 1 M 117 -> 110 us, 245 k mixed 22.6 -> 20.2 us.
+  // us; SST 1 M 117 -> 110 us, 258 k mixed 22.6 -> 20.2 us.
   int fe[4], nb[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) fe[i] = m.cf[i * nc + c];
@@ -939,7 +939,7 @@ __device__ __forceinline__ void cell_terms(const DevMesh &m, const DevState &s, 
   // for Euler).  Bound by these two latencies on small meshes, by its
   // traffic on large ones.  Measured: Euler 20 k cells 10.4 -> 3.6 us, 106 k
   // 20.7 -> 5.9 us; laminar 100 k (batch) 10.0 -> 8.0 us; SST 1 M 99.9 ->
-  // 97.3 us, 245 k mixed 16.7 -> 14.4 us.
+  // 97.3 us, 258 k mixed 16.7 -> 14.4 us.
   int fs[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) fs[i] = m.cf[i * nc + c];
@@ -2439,10 +2439,13 @@ static int sweep_launches(const usg_ctx *c) {
 }
 
 // A sweep launch takes 3.5-6 us however few cells it holds, a level of up to
-// kLevelGroups * kLevelCells cells in k_levels a tenth of that, so the narrow last levels of
-// the two sweeps go to k_levels when that replaces at least kLevelMin
-// launches (which repay its own four).  A level is narrow up to kLevelWidth
-// cells of a case: two rounds of chunks, where the launch is about as fast.
+// kLevelCells cells in k_levels a tenth of that, so the narrow last levels of
+// the two sweeps go to k_levels when that replaces at least kLevelMin launches
+// (which repay its own four: 3 x 4 cells, 12 launches, 58 -> 46 us an iteration).
+// A level is narrow up to kLevelWidth cells of a case, two rounds of chunks,
+// which take 2.9 us where a launch takes 5.2 (Euler, 512 x 600 quads in row
+// order, an iteration 17.1 -> 6.4 ms; 520 x 600 keep their launches, 11.5 ms).
+// Their ring is 64 KB of LDS, for SST 96 KB.
 constexpr int kLevelMin = 12, kLevelWidth = 8 * kLevelCells;
 
 // Lets k_levels take `limit` bytes of LDS, the device's most: what is set holds
@@ -3086,8 +3089,10 @@ static int ctx_setup(usg_ctx *c, usg_ctx **out) {
   // 4 MB) and a face's cells are far apart in the numbering (colour blocks):
   // SST 1 M 148 -> 136 us, 512 k 72.8 -> 70.7 us, Euler 258 k 19.8 -> 18.2
   // us.  Below, a chunk's load costs more than it saves (SST 128 k 19.7 ->
-  // 20.0 us), and in rows of cells the order as it is serves (SST 200 k in
-  // rows 35.9 -> 38.1 us).
+  // 20.0 us).  The line itself matters little: on squares of 177 k to 518 k
+  // quads the two forms are within 3 % of one another in every flow (SST 250 k
+  // 43.7 us with, 43.8 without; 314 k 55.2 / 55.0).  In rows of cells the order
+  // as it is serves (SST 200 k in rows 35.9 -> 38.1 us).
   const size_t gathered = 4 * sizeof(double) + 12 * (c->prm.precision == USG_MIXED ? sizeof(float) : sizeof(double));
   if (c->sweep_ident && nc * gathered > 32000000)
     CK(upload(c, &c->d_face_chunks, h.face_chunks.data(), h.face_chunks.size()));
