@@ -229,8 +229,8 @@ __device__ __forceinline__ void put4(bf16 *rows, int ld, bf16 *op, int p0, int N
 // and back.  A layer's weights come from L2 into registers while the previous
 // layer's activation is in work.
 // Bound by the vector instructions of the SiLU and its derivative: they issue
-// in 42 % of the SIMDs' cycles in training, whose two waves per SIMD wait for
-// data or a barrier a third of their time, and in 67 % in inference; matrix
+// in 40 % of the SIMDs' cycles in training, whose two waves per SIMD wait for
+// data or a barrier a third of their time, and in 63 % in inference; matrix
 // instructions take 14 and 18 %.  Measured at 8 x 256 on 16384 points: 116 us,
 // against 350 us for a launch per product (and one each for the batch, the loss
 // and the last layer).  Inference of 12576 points takes 36 us, against 98 us, with the two
