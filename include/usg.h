@@ -157,7 +157,8 @@ int usg_lusgs_step(usg_ctx *ctx, int n, double *res_hist);
  * res_hist as for usg_lusgs_step (the stage-0 residual of each step). */
 int usg_rk5_step(usg_ctx *ctx, int n, double *res_hist);
 
-/* Copy a field to the host (AoS layout of the reference); count = elements. */
+/* Copy a field to the host (AoS layout of the reference); count = elements.
+ * Threads may read fields of one context side by side. */
 int usg_get_field(usg_ctx *ctx, int field, double *out, long count);
 /* ||R_rho / V||_2 of the last residual (the convergence norm), out[ncases]. */
 int usg_res_l2(usg_ctx *ctx, double *out);
